@@ -1703,64 +1703,110 @@ extern "C" hipError_t gpu_increment_decode_state_on_stream(int* d_state, hipStre
 // for the tile, l = l * alpha + sum of the unrounded exps, O = O * alpha +
 // P V (fp32 accumulate), out = O / l.
 //
-// Workgroup: 4 waves over 128 queries of one head (wave w: queries
-// q0 + 32w ..), sharing the head's K tile ([key][dim]) and transposed V
-// tile ([dim][key]) in LDS.  Each wave computes S^T = K Q^T (two 32x32
-// blocks of v_mfma_f32_32x32x16_f16, Q^T from registers), so a lane owns
-// one query column: the row max / sum are in-lane plus one exchange with
-// lane ^ 32, alpha is a per-lane scale of the O^T accumulators, and the
-// accumulator values of P feed the B operand of O^T = V^T P^T directly --
-// the key order they come in is matched by the order the V^T operand is
-// read in.  exp(x - m) is evaluated as 2^(x log2 e - m log2 e) (one
-// v_exp_f32; within a few fp32 ulps of expf, P is rounded to fp16 anyway),
-// the causal mask is applied only on the tiles that reach past a wave's
-// first query, and O is rescaled only when some lane's maximum moved.  The
-// next K / V tile is loaded into registers while the current one is used;
-// V is written transposed as 32-bit key pairs, its keys permuted (bits 2
-// and 3 swapped) so that the 8 keys of an operand are one 16-byte read, and
-// XOR-swizzled by 8 ((dim / 8) % 8) so that the 16 threads writing one key
-// pair (rows 8 apart) hit different banks.  Measured at 512 positions, 32
-// heads, fp32 output: 26.5 us before these changes (and one wave per SIMD,
-// the mask on diagonal tiles only), 17.4 after, the same bits.
+// Each wave owns a unit: 32 queries of one head.  It computes S^T = K Q^T
+// (two 32x32 blocks of v_mfma_f32_32x32x16_f16, Q^T in registers), so a lane
+// owns one query column: the row max is in-lane plus one exchange with
+// lane ^ 32, the row sum is kept per half wave and added at the end, and the
+// accumulator values of P feed the B operand of O^T = V^T P^T directly -- the
+// key order they come in is matched by the order the V^T operand is read in.
+// A workgroup's units run over (query block, head of the KV head's group),
+// heads fastest: the waves share their K / V tiles and stay within a query
+// block or two of each other, whatever the group size.  K / V tiles arrive by
+// LDS DMA in rows as they lie in memory, double buffered, one barrier per
+// tile; V is transposed by its reads (ds_read_b64_tr_b16).  The longest query
+// blocks start first, and a KV head's workgroups fall on one XCD when the KV
+// heads are a multiple of 8 (its K / V then stay in that L2).
+//
+// Bound: a 64-key tile is 32 MFMAs (1024 matrix cycles) against ~900 cycles
+// of softmax VALU per wave (32 v_exp_f32 at quarter rate, and an fma, an add
+// and half a max and a conversion per score), which overlap only across the
+// two waves of a SIMD.  32 / 8 heads, causal, fp16 output, graph replays, us
+// (TFLOP/s): 512 positions 17.2 -> 11.1, 1024 31.3 -> 23.2, 2048 110 -> 50
+// (686), 4096 420 -> 149 (920), 8192 1341 -> 552 (996).  Before: one wave
+// per SIMD over 128 queries of one head, tiles through registers, V
+// transposed by 2-byte LDS stores.
 namespace rf {
 
+typedef _Float16 h4 __attribute__((ext_vector_type(4)));
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
+typedef short s4 __attribute__((ext_vector_type(4)));
 typedef float f16v __attribute__((ext_vector_type(16)));
 
 constexpr int kAttD = 128;
-constexpr int kKStr = kAttD + 8;     // K tile row stride (halves)
-constexpr int kVStr = 64 + 8;        // V^T tile row stride (halves)
+constexpr uint32_t kAttRow = 2 * kAttD;          // bytes of a K / V row in LDS
+constexpr uint32_t kAttTile = 64 * kAttRow;      // one 64-key tile of K or of V
 
+// NW waves as NW / KS units times KS key groups: group g takes the tiles
+// t % KS == g and the groups' partial (m, l, O) are merged through LDS (more
+// waves and a shorter walk per unit when the units are few).  VE: the V
+// operands are read before the softmax (64 VGPRs; in flight during it).
 // OUT = float, or uint16_t: fp16 bits of the fp32 output (round to nearest
 // even), the operand a GEMM on fp16 activations reads
-// One wave per SIMD (waves_per_eu 1): the whole register file for the
-// accumulators and the prefetched tile (measured 22.8 against 26.5 us at 512
-// positions, 32 heads).
-template <int NWQ, typename OUT>
-__global__ __launch_bounds__(64 * NWQ) __attribute__((amdgpu_waves_per_eu(1, 1))) void rf_attn_prefill_kernel(const _Float16* __restrict__ Q,
-                                                              const _Float16* __restrict__ K,
-                                                              const _Float16* __restrict__ V, OUT* __restrict__ O,
-                                                              int seq, int nq, int nkv, int causal, float scale) {
-    __shared__ __align__(16) _Float16 ks[64 * kKStr];
-    __shared__ __align__(16) _Float16 vt[kAttD * kVStr];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int head = blockIdx.y;
-    const int kvh = head / (nq / nkv);
-    const int qb = blockIdx.x * 32 * NWQ;
-    const int q0 = qb + 32 * wave;
+template <int NW, int KS, bool VE, typename OUT>
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW / 4)))
+void rf_attn_prefill_kernel(const _Float16* __restrict__ Q, const _Float16* __restrict__ K,
+                            const _Float16* __restrict__ V, OUT* __restrict__ O, int seq, int nq, int nkv, int group,
+                            uint32_t group_inv, int units, int last_wg, int causal, float scale) {
+    constexpr int U = NW / KS;                   // (query block, head) units per workgroup
+    __shared__ __align__(1024) uint8_t lds[2 * KS * 2 * kAttTile];   // [buffer][key group][K, V]
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int hi = lane >> 5, col = lane & 31;
-    const size_t qrow = (size_t)nq * kAttD, kvrow = (size_t)nkv * kAttD;
-    const bool active = q0 < seq;
+    const int kvh = blockIdx.x, wg = last_wg - (int)blockIdx.y;
+    const int ks = wave / U;
+    const int unit = wg * U + wave % U;
+    const bool active = unit < units;
+    const int uc = min(unit, units - 1);
+    auto block_of = [&](int u) {                 // u / group
+        return group == 1 ? u : group_inv ? (int)__umulhi((uint32_t)u, group_inv) : u / group;
+    };
+    const int head = kvh * group + uc - block_of(uc) * group;
+    const int q0 = 32 * block_of(uc);
+    const uint32_t kvrow = (uint32_t)nkv * kAttRow;          // bytes
+    const size_t qrow = (size_t)nq * kAttD;
 
-    // Q^T operands of this lane's query: dims 16 ks + 8 hi .. + 7
-    h8 qf[8];
+    const int last_q0 = 32 * block_of(min(wg * U + U - 1, units - 1));
+    const int ntiles = causal ? last_q0 / 64 + 1 : seq / 64;
+    const int wave_tiles = !active ? 0 : causal ? q0 / 64 + 1 : seq / 64;
+
+    // LDS DMA: instruction j of a tile moves rows 4 j .. 4 j + 3 (lane: row
+    // lane / 16, 16-byte slot lane % 16); a row's pieces are permuted by the
+    // source address: K piece p of row r in slot p ^ (r % 16), V piece p of row
+    // r in slot p ^ 4 (r % 4)
+    constexpr int NJ = 16 / NW;                  // instructions per wave, tile and matrix
+    static_assert(NW % 4 == 0 && 16 % NW == 0, "a wave's rows keep their residue mod 16 from one instruction to the next");
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)lds;
+    const int dr = lane >> 4, ds = lane & 15;
+    const uint32_t koff = (uint32_t)(4 * wave + dr) * kvrow + 16u * (uint32_t)(ds ^ ((4 * wave + dr) & 15));
+    const uint32_t voff = (uint32_t)(4 * wave + dr) * kvrow + 16u * (uint32_t)(ds ^ (4 * dr));
+    const uint8_t* kbase = reinterpret_cast<const uint8_t*>(K) + (size_t)kvh * kAttRow;
+    const uint8_t* vbase = reinterpret_cast<const uint8_t*>(V) + (size_t)kvh * kAttRow;
+    auto stage = [&](int it, int buf) {
 #pragma unroll
-    for (int ks_ = 0; ks_ < 8; ++ks_) {
-        if (active)
-            qf[ks_] = *reinterpret_cast<const h8*>(Q + (size_t)(q0 + col) * qrow + (size_t)head * kAttD + 16 * ks_ +
-                                                   8 * hi);
-        else
-            qf[ks_] = h8{};
+        for (int k = 0; k < KS; ++k) {
+            const int t = KS * it + k;
+            if (t >= ntiles) break;
+            const uint32_t dst = lds0 + (uint32_t)((buf * KS + k) * 2) * kAttTile + 1024u * (uint32_t)wave;
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) {
+                const size_t off = (size_t)(64 * t + 4 * NW * j) * kvrow;
+                lds_dma16(__builtin_amdgcn_readfirstlane(dst + 1024u * NW * j), koff, kbase + off);
+                lds_dma16(__builtin_amdgcn_readfirstlane(dst + kAttTile + 1024u * NW * j), voff, vbase + off);
+            }
+        }
+    };
+    stage(0, 0);
+
+    // Q^T operands of this lane's query: dims 16 k + 8 hi .. + 7; a negative
+    // scale moves its sign here (exact), so that the largest S has the largest weight
+    typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+    const uint32_t sign = scale < 0.0f ? 0x80008000u : 0u;
+    h8 qf[8];
+    // (1e-30: a scale of zero keeps every weight at one and the masked ones at zero)
+    const float scale2 = fmaxf(fabsf(scale) * 1.4426950408889634f, 1e-30f);   // log2 e
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        const u4 w = *reinterpret_cast<const u4*>(Q + (size_t)(q0 + col) * qrow + (size_t)head * kAttD + 16 * k + 8 * hi);
+        qf[k] = __builtin_bit_cast(h8, w ^ sign);
     }
     f16v o[4];
 #pragma unroll
@@ -1769,140 +1815,134 @@ __global__ __launch_bounds__(64 * NWQ) __attribute__((amdgpu_waves_per_eu(1, 1))
         for (int e = 0; e < 16; ++e) o[b][e] = 0.0f;
     float m = kNegMax, l = 0.0f;
     const int query = q0 + col;
-    const float scale2 = scale * 1.4426950408889634f;   // log2 e
 
-    const int wg_last_q = min(qb + 32 * NWQ - 1, seq - 1);
-    const int ntiles = causal ? wg_last_q / 64 + 1 : seq / 64;
-    const int wave_tiles = causal ? (q0 + 31) / 64 + 1 : seq / 64;
-    // K / V tiles: thread chunk i = key c >> 4, dims (c & 15) * 8, c = tid +
-    // 64 NWQ i; tile t + 1 is loaded into registers while tile t is used
-    // (V: chunks 2 p, 2 p + 1 are keys 2 (tid / 16 + 4 NWQ p) and the next, so
-    // the transposed tile takes them as one 32-bit key pair per dim)
-    constexpr int NCH = 16 / NWQ;
-    auto vkey = [&](int i) { return 2 * ((tid >> 4) + 4 * NWQ * (i >> 1)) + (i & 1); };
-    auto vpos = [](int k) { return (k & ~12) | ((k & 4) << 1) | ((k & 8) >> 1); };
-    h8 kr[NCH], vr[NCH];
-    auto tile_load = [&](int t0) {
+    // operand addresses: K lane (row col, piece 2 k + hi) in slot piece ^ (col %
+    // 16); V by transposing reads: lanes 16 g + i read keys 4 (g / 2) + i / 4,
+    // dims 32 bd + 16 (g % 2) + 4 (i % 4) .. + 3 and receive 4 keys of dim 32 bd + col
+    const uint32_t ka = lds0 + (uint32_t)col * kAttRow + 16u * (uint32_t)(hi ^ (col & 15));
+    const int i16 = lane & 15;
+    uint32_t va[4];
 #pragma unroll
-        for (int i = 0; i < NCH; ++i) {
-            const int c = tid + 64 * NWQ * i;
-            const int key = c >> 4, d8 = (c & 15) * 8;
-            kr[i] = *reinterpret_cast<const h8*>(K + (size_t)(t0 + key) * kvrow + (size_t)kvh * kAttD + d8);
-            vr[i] = *reinterpret_cast<const h8*>(V + (size_t)(t0 + vkey(i)) * kvrow + (size_t)kvh * kAttD + d8);
-        }
-    };
-    if (ntiles > 0) tile_load(0);
-    for (int t = 0; t < ntiles; ++t) {
-        const int t0 = 64 * t;
-        __syncthreads();   // previous tile's reads done
-        // K tile: 64 keys x 128 dims, 16-byte chunks; V tile transposed
-#pragma unroll
-        for (int i = 0; i < NCH; ++i) {
-            const int c = tid + 64 * NWQ * i;     // 0..1023
-            const int key = c >> 4, d8 = (c & 15) * 8;
-            const h8 kv = kr[i];
-            *reinterpret_cast<h8*>(&ks[key * kKStr + d8]) = kv;
-        }
-        // V transposed: key k of a row at position vpos(k) ^ 8 ((d / 8) % 8),
-        // vpos swapping bits 2 and 3 of the key (so the 8 keys an MFMA operand
-        // takes, k .. k + 3 and k + 8 .. k + 11 for k % 8 = 0 or 4, are one
-        // aligned 16-byte run), the XOR spreading the 16 threads of a key pair,
-        // whose rows are 8 apart, over the banks
-#pragma unroll
-        for (int pi = 0; pi < NCH / 2; ++pi) {
-            const int d8 = (tid & 15) * 8, k0 = vkey(2 * pi);
-            const int sw = 8 * (tid & 7);
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-                const h2 pr = {vr[2 * pi][j], vr[2 * pi + 1][j]};
-                *reinterpret_cast<h2*>(&vt[(d8 + j) * kVStr + (vpos(k0) ^ sw)]) = pr;
-            }
-        }
-        if (t + 1 < ntiles) tile_load(t0 + 64);
-        __syncthreads();
-        if (!active || t >= wave_tiles) continue;
+    for (int bd = 0; bd < 4; ++bd)
+        va[bd] = lds0 + kAttTile + (uint32_t)(4 * hi + (i16 >> 2)) * kAttRow + 64u * (uint32_t)(bd ^ (i16 >> 2)) +
+                 16u * (uint32_t)(2 * ((lane >> 4) & 1) + ((i16 & 3) >> 1)) + 8u * (uint32_t)(i16 & 1);
+    typedef __attribute__((address_space(3))) const h8* lds_h8;
+    typedef __attribute__((address_space(3))) s4* lds_s4;
+
+    const int iters = (ntiles + KS - 1) / KS;
+    for (int it = 0; it < iters; ++it) {
+        const int buf = it & 1;
+        // this wave's share of the tiles has landed; past the barrier everyone's
+        // has, and the other buffer's reads are done
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        lds_barrier();
+        if (it + 1 < iters) stage(it + 1, buf ^ 1);
+        const int t = KS * it + ks, t0 = 64 * t;
+        if (t >= wave_tiles) continue;
+        const uint32_t tb = (uint32_t)((buf * KS + ks) * 2) * kAttTile;
 
         // S^T = K Q^T: blocks b = keys 32 b .. + 31
         f16v s[2];
 #pragma unroll
-        for (int b = 0; b < 2; ++b) {
+        for (int b = 0; b < 2; ++b)
 #pragma unroll
             for (int e = 0; e < 16; ++e) s[b][e] = 0.0f;
 #pragma unroll
-            for (int ks_ = 0; ks_ < 8; ++ks_) {
-                const h8 a = *reinterpret_cast<const h8*>(&ks[(32 * b + col) * kKStr + 16 * ks_ + 8 * hi]);
-                s[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, qf[ks_], s[b], 0, 0, 0);
-            }
+        for (int k = 0; k < 8; ++k) {
+            const uint32_t kk = (ka ^ (32u * k)) + tb;
+#pragma unroll
+            for (int b = 0; b < 2; ++b)
+                s[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(*(lds_h8)(kk + 32u * b * kAttRow), qf[k], s[b], 0, 0, 0);
         }
-        // scale (in the log2 domain: exp(x - m) = 2^(x log2 e - m log2 e), one
-        // v_exp_f32 each), mask (only a tile that reaches past the wave's first
-        // query holds keys to mask: a branch of its own, so the other tiles
-        // carry no compare and select per element), tile max
+        // V^T operand (k-step j, dims 32 bd ..): lane (dim 32 bd + col) takes keys in
+        // the order P's accumulators hold them, 16 j + 4 hi + {0..3, 8..11}
+        auto v_frag = [&](int j, int bd) {
+            const uint32_t vv = va[bd] + tb + 16u * j * kAttRow;
+            const h4 a0 = __builtin_bit_cast(h4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4)vv));
+            const h4 a1 = __builtin_bit_cast(h4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4)(vv + 8u * kAttRow)));
+            return __builtin_shufflevector(a0, a1, 0, 1, 2, 3, 4, 5, 6, 7);
+        };
+        h8 vf[16];
+        if constexpr (VE) {
+#pragma unroll
+            for (int i = 0; i < 16; ++i) vf[i] = v_frag(i >> 2, i & 3);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        // only a tile that reaches past the wave's first query holds keys to mask
+        if (causal && t0 + 63 > q0) {
+#pragma unroll
+            for (int b = 0; b < 2; ++b)
+#pragma unroll
+                for (int e = 0; e < 16; ++e)
+                    if (t0 + 32 * b + 8 * (e >> 2) + 4 * hi + (e & 3) > query) s[b][e] = kNegMax;
+        }
         float tmax = kNegMax;
-        const bool diag = causal && t0 + 63 > q0;
-        if (diag) {
 #pragma unroll
-            for (int b = 0; b < 2; ++b)
+        for (int b = 0; b < 2; ++b)
 #pragma unroll
-                for (int e = 0; e < 16; ++e) {
-                    float v = s[b][e] * scale2;
-                    const int key = t0 + 32 * b + 8 * (e >> 2) + 4 * hi + (e & 3);
-                    if (key > query) v = kNegMax;
-                    s[b][e] = v;
-                    tmax = fmaxf(tmax, v);
-                }
-        } else {
+            for (int e = 0; e < 16; ++e) tmax = fmaxf(tmax, s[b][e]);
+        tmax = fmaxf(tmax, __shfl_xor(tmax, 32)) * scale2;
+        // O is rescaled only where some lane's maximum moved.  (A maximum left behind
+        // by up to 2^8 saves 6 % of the time, but then a row's largest weight is no
+        // longer exactly one and peaked rows lose half their precision.)
+        if (__builtin_amdgcn_ballot_w64(tmax > m)) {
+            const float m_new = fmaxf(m, tmax);
+            const float alpha = __builtin_amdgcn_exp2f(m - m_new);
+            m = m_new;
+            l *= alpha;
 #pragma unroll
-            for (int b = 0; b < 2; ++b)
+            for (int b = 0; b < 4; ++b)
 #pragma unroll
-                for (int e = 0; e < 16; ++e) {
-                    const float v = s[b][e] * scale2;
-                    s[b][e] = v;
-                    tmax = fmaxf(tmax, v);
-                }
+                for (int e = 0; e < 16; ++e) o[b][e] *= alpha;
         }
-        tmax = fmaxf(tmax, __shfl_xor(tmax, 32));
-        const float m_new = fmaxf(m, tmax);
-        const float alpha = __builtin_amdgcn_exp2f(m - m_new);
+        // exp(x - m) as 2^(s scale log2 e - m log2 e): one fma, one v_exp_f32
         float rs = 0.0f;
         h8 p[4];   // B operands, k-step j = (block j / 2, keys 16 (j % 2) ..)
 #pragma unroll
         for (int b = 0; b < 2; ++b)
 #pragma unroll
             for (int e = 0; e < 16; ++e) {
-                const float ex = __builtin_amdgcn_exp2f(s[b][e] - m_new);
+                const float ex = __builtin_amdgcn_exp2f(__builtin_fmaf(s[b][e], scale2, -m));
                 rs += ex;
                 p[2 * b + (e >> 3)][e & 7] = (_Float16)ex;
             }
-        rs += __shfl_xor(rs, 32);
-        l = l * alpha + rs;
-        m = m_new;
-        // rescale O only where some lane's maximum moved (alpha == 1 elsewhere:
-        // multiplying by it changes nothing)
-        if (__builtin_amdgcn_ballot_w64(alpha != 1.0f)) {
+        l += rs;
+        // O^T += V^T P^T
 #pragma unroll
-            for (int b = 0; b < 4; ++b)
+        for (int j = 0; j < 4; ++j)
 #pragma unroll
-                for (int e = 0; e < 16; ++e) o[b][e] *= alpha;
-        }
-        // O^T += V^T P^T: A operand lane (dim = 32 bd + col) keys of k-step j in
-        // the accumulator order: 32 (j/2) + 16 (j%2) + 4 hi + {0..3, 8..11}
+            for (int bd = 0; bd < 4; ++bd)
+                o[bd] = __builtin_amdgcn_mfma_f32_32x32x16_f16(VE ? vf[4 * j + bd] : v_frag(j, bd), p[j], o[bd], 0, 0, 0);
+    }
+    // the key groups' partial (m, l, O): group 1 hands its own to group 0
+    static_assert(KS <= 2, "one partner per unit");
+    if constexpr (KS == 2) {
+        if (ntiles > 1) {
+            lds_barrier();
+            float* part = reinterpret_cast<float*>(lds) + (wave % U) * (66 * 64) + lane;
+            if (ks > 0) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int kb = 32 * (j >> 1) + 16 * (j & 1) + 4 * hi;
+                for (int b = 0; b < 4; ++b)
 #pragma unroll
-            for (int bd = 0; bd < 4; ++bd) {
-                // row d = 32 bd + col, keys kb .. kb + 3 and kb + 8 .. kb + 11: the
-                // 16-byte run at vpos(kb) under the row's swizzle 8 ((d / 8) % 8)
-                const int sw = 8 * ((4 * bd + (col >> 3)) & 7);
-                const _Float16* vrow = &vt[(32 * bd + col) * kVStr];
-                const h8 a = *reinterpret_cast<const h8*>(vrow + (vpos(kb) ^ sw));
-                o[bd] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, p[j], o[bd], 0, 0, 0);
+                    for (int e = 0; e < 16; ++e) part[(16 * b + e) * 64] = o[b][e];
+                part[64 * 64] = m;
+                part[65 * 64] = l;
+            }
+            lds_barrier();
+            if (ks == 0) {
+                const float mk = part[64 * 64], mn = fmaxf(m, mk);
+                const float f0 = __builtin_amdgcn_exp2f(m - mn), f1 = __builtin_amdgcn_exp2f(mk - mn);
+#pragma unroll
+                for (int b = 0; b < 4; ++b)
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) o[b][e] = o[b][e] * f0 + part[(16 * b + e) * 64] * f1;
+                l = l * f0 + part[65 * 64] * f1;
             }
         }
+        if (ks > 0) return;
     }
     if (!active) return;
+    l += __shfl_xor(l, 32);                      // each half wave summed its own keys
     const float inv_l = l > 0.0f ? 1.0f / l : 0.0f;
     OUT* orow = O + (size_t)query * qrow + (size_t)head * kAttD;
 #pragma unroll
@@ -1919,6 +1959,21 @@ __global__ __launch_bounds__(64 * NWQ) __attribute__((amdgpu_waves_per_eu(1, 1))
 
 }  // namespace rf
 
+template <int NW, int KS, bool VE, typename OUT>
+static void attn_prefill_go(const void* Q, const void* K, const void* V, OUT* O, int seq_len, int nq, int nkv,
+                            int causal, float scale, hipStream_t stream) {
+    const int group = nq / nkv, units = group * (seq_len / 32), nwg = (units + NW / KS - 1) / (NW / KS);
+    // unit / group as the high word of a product: exact for units * group < 2^32
+    const bool small = group > 1 && (unsigned long long)units * group < (1ull << 32);
+    const uint32_t inv = small ? (uint32_t)(((1ull << 32) + group - 1) / group) : 0;
+    constexpr int kGridY = 65535;
+    for (int w = nwg; w > 0; w -= kGridY)        // longest query blocks first
+        hipLaunchKernelGGL((rf::rf_attn_prefill_kernel<NW, KS, VE, OUT>), dim3(nkv, w < kGridY ? w : kGridY),
+                           dim3(64 * NW), 0, stream, static_cast<const _Float16*>(Q), static_cast<const _Float16*>(K),
+                           static_cast<const _Float16*>(V), O, seq_len, nq, nkv, group, inv, units, w - 1, causal,
+                           scale);
+}
+
 template <typename OUT>
 static hipError_t attn_prefill(const void* Q, const void* K, const void* V, OUT* O, int seq_len, int num_q_heads,
                                int num_kv_heads, int causal, float scale, hipStream_t stream) {
@@ -1927,10 +1982,21 @@ static hipError_t attn_prefill(const void* Q, const void* K, const void* V, OUT*
     if (seq_len <= 0 || seq_len % 64 != 0) return hipErrorInvalidValue;
     if ((reinterpret_cast<uintptr_t>(Q) | reinterpret_cast<uintptr_t>(K) | reinterpret_cast<uintptr_t>(V)) & 15u)
         return hipErrorInvalidValue;
-    // four waves (128 queries) per workgroup: measured faster than two
-    hipLaunchKernelGGL((rf::rf_attn_prefill_kernel<4, OUT>), dim3((seq_len + 127) / 128, num_q_heads), dim3(256), 0,
-                       stream, static_cast<const _Float16*>(Q), static_cast<const _Float16*>(K),
-                       static_cast<const _Float16*>(V), O, seq_len, num_q_heads, num_kv_heads, causal, scale);
+    // 32-query units over the CUs (64 KB of LDS per key group, so at most two
+    // workgroups on a CU): two units and two key groups a workgroup while those
+    // workgroups are one a CU or fewer (512 positions, 32 heads: 10.5 us, four
+    // units 13.5, eight units unsplit 19.2), eight unsplit units where they come
+    // to two a CU, so that long and short query blocks even out (4096 positions:
+    // 143 us against 157 with four units and two key groups), four units and two
+    // key groups between (2048: 47 against 61 and 57; these figures from one run
+    // of a form with a cheaper rescale, all routes alike)
+    const long long units = (long long)num_q_heads * (seq_len / 32), cus = rf::device_cu_count();
+    if (units <= 2 * cus)
+        attn_prefill_go<4, 2, true>(Q, K, V, O, seq_len, num_q_heads, num_kv_heads, causal, scale, stream);
+    else if (units < 16 * cus)
+        attn_prefill_go<8, 2, false>(Q, K, V, O, seq_len, num_q_heads, num_kv_heads, causal, scale, stream);
+    else
+        attn_prefill_go<8, 1, true>(Q, K, V, O, seq_len, num_q_heads, num_kv_heads, causal, scale, stream);
     return hipGetLastError();
 }
 
