@@ -15,14 +15,14 @@
 //    of the CUs): 4 waves, each weight dequantised once per 256 rows of A,
 //    A and the weight ring by LDS DMA.
 //  * rf_gemm_q4k_f16s_kernel (Q4_K otherwise) and rf_gemm_q6k_f16a_kernel
-//    (Q6_K, K % 2048 == 0): 8 waves over 64- or 128-row x 64-column tiles, K
+//    (Q6_K from K = 768): 8 waves over 64- or 128-row x 64-column tiles, K
 //    sliced over waves and added through LDS; when the tiles leave at least
 //    half the CUs idle, K is also split over workgroups whose partial tiles
 //    rf_gemm_split_reduce_kernel adds in split order.
 // Every output is one fixed-order sum: no float atomics, the same bits on
-// every run.  When no staging memory is free for the stream (or Q6_K rows are
-// not 16-byte aligned) the fp32-activation kernels run, one workgroup per
-// tile:
+// every run.  When no staging memory is free for the stream (or Q6_K weights
+// are not 16-byte aligned, or K is 256 or 512 with them) the fp32-activation
+// kernels run, one workgroup per tile:
 //  * rf_gemm_qk_sq_kernel (N % 256 == 0, K % 512 == 0, and 256 x 256 or
 //    128 x 128 tiles that come to about one workgroup per CU): 2 x 2 waves,
 //    each weight dequantised once per workgroup into an LDS B tile shared by
@@ -1876,8 +1876,11 @@ __global__ __launch_bounds__(kF16aThreads) void rf_gemm_q4k_f16a_kernel(const ui
 // 240-byte LDS row (60 dwords: the 32 rows of a read fall on 8 banks, 4-way),
 // loaded by 16-byte LDS DMA (16 instructions per stage: the DMA costs per
 // instruction, not per byte).  Three stages: super-block
-// sb + 2 loads while sb is used.  K % 2048 == 0 keeps the last window of a
-// row inside it.  A arrives as in rf_gemm_q4k_f16a_kernel
+// sb + 2 loads while sb is used.  With K % 2048 == 0 every row starts at a
+// 16-byte piece; for other K (ANY) the piece and the phase are taken per row.
+// A tile's first row (n0 % 64 == 0) starts at a piece either way, and the
+// matrix ends at one (N % 64 == 0), so no window leaves it: its last block
+// sits at byte 14 of its window and ends with it.  A arrives as in rf_gemm_q4k_f16a_kernel
 // (16-byte LDS DMA, XOR-swizzled 128-byte rows), seven chunk buffers deep:
 // a DMA gets four chunks to land.
 //
@@ -1951,7 +1954,10 @@ __device__ __forceinline__ u32x2 q6a_dq4(uint32_t qb, float S24, float nO) {
 
 // Tile v of the launch (after the XCD remap); lds: the kLds-byte LDS block.
 
-template <bool ACC, int FMR = 4>
+// ANY: K any multiple of 256, so a row starts anywhere in a 16-byte piece and
+// a lane's window phase depends on its row; otherwise K % 2048 == 0 and every
+// row starts at a piece.
+template <bool ACC, int FMR = 4, bool ANY = false>
 __device__ __forceinline__ void q6a_wg(const uint16_t* __restrict__ A, const uint8_t* __restrict__ W,
                                        float* __restrict__ D, int M, int N, int K, int v, uint8_t* lds,
                                        KSplit sp = KSplit{1, nullptr}) {
@@ -1988,17 +1994,21 @@ __device__ __forceinline__ void q6a_wg(const uint16_t* __restrict__ A, const uin
     // piece 13) ----------------------------------------------------------------
     const uint8_t* w_tile = W + (size_t)n0 * row_bytes;
     constexpr int kRPW = kQ6aRingInstr / 8;   // 2 per wave per super-block
-    uint32_t roff[kRPW];
+    uint32_t roff[kRPW], rpc[kRPW];
 #pragma unroll
     for (int t = 0; t < kRPW; ++t) {
         const int i = 64 * (wave + 8 * t) + lane;
         const int r = min(i / 15, 63), pc = i < 960 ? min(i % 15, 13) : 13;
-        roff[t] = (uint32_t)r * row_bytes + 16u * (uint32_t)pc;
+        roff[t] = (uint32_t)r * row_bytes + (ANY ? 0u : 16u * (uint32_t)pc);
+        rpc[t] = 16u * (uint32_t)pc;
     }
     auto w_dma1 = [&](int t, int sb, int slot) {
         const int s = sb0 + min(sb, nsb - 1);
-        lds_dma16(ring_lds0 + (uint32_t)slot * kQ6aStage + 1024u * (uint32_t)(wave + 8 * t), roff[t],
-                  w_tile + (size_t)((s * kQ6KBytes) & ~15));
+        const uint32_t dst = ring_lds0 + (uint32_t)slot * kQ6aStage + 1024u * (uint32_t)(wave + 8 * t);
+        if constexpr (ANY)
+            lds_dma16(dst, ((roff[t] + (uint32_t)(s * kQ6KBytes)) & ~15u) + rpc[t], w_tile);
+        else
+            lds_dma16(dst, roff[t], w_tile + (size_t)((s * kQ6KBytes) & ~15));
     };
 
     // ---- A: instruction gi = kAPW wave + g covers rows 8 gi + L / 8 of the
@@ -2023,15 +2033,25 @@ __device__ __forceinline__ void q6a_wg(const uint16_t* __restrict__ A, const uin
     // per-super-block factors d * 2^24 and -32 d, and the chunk's sub-block
     // scale -------------------------------------------------------------------
     const int brow = 32 * cg + col;
+    const int row_phase = ANY ? 2 * brow * nsb_row : 0;       // n0 % 64 == 0 adds a multiple of 16
+    auto block_off = [&](int sb) { return (row_phase + 2 * (sb0 + sb)) & 15; };
     uint32_t rql[2], rqh[2];
     auto raw_read = [&](int n, int sb) {
-        const int off = (2 * (sb0 + sb)) & 15;
+        const int off = block_off(sb);
         const uint8_t* rowp = ring + (sb % G::kRS) * kQ6aStage + brow * kQ6aRowB;
         const int oql = off + 64 * n + 16 * ks + 8 * h;
         const int oqh = off + 128 + 32 * n + 16 * (ks & 1) + 8 * h;
         const uint32_t* pl = reinterpret_cast<const uint32_t*>(rowp + (oql & ~3));
         const uint32_t* ph = reinterpret_cast<const uint32_t*>(rowp + (oqh & ~3));
-        if ((sb0 + sb) & 1) {
+        if constexpr (ANY) {
+            const uint32_t l0 = pl[0], l1 = pl[1], l2 = pl[2];
+            const uint32_t h0 = ph[0], h1 = ph[1], h2 = ph[2];
+            const uint32_t sh = (uint32_t)(off & 2) * 8;
+            rql[0] = __builtin_amdgcn_alignbit(l1, l0, sh);
+            rql[1] = __builtin_amdgcn_alignbit(l2, l1, sh);
+            rqh[0] = __builtin_amdgcn_alignbit(h1, h0, sh);
+            rqh[1] = __builtin_amdgcn_alignbit(h2, h1, sh);
+        } else if ((sb0 + sb) & 1) {
             const uint32_t l0 = pl[0], l1 = pl[1], l2 = pl[2];
             const uint32_t h0 = ph[0], h1 = ph[1], h2 = ph[2];
             rql[0] = __builtin_amdgcn_alignbit(l1, l0, 16);
@@ -2048,14 +2068,14 @@ __device__ __forceinline__ void q6a_wg(const uint16_t* __restrict__ A, const uin
     float d24 = 0.0f, dm32 = 0.0f;
     int scb = 0;
     auto d_read = [&](int sb) {
-        const int off = (2 * (sb0 + sb)) & 15;
+        const int off = block_off(sb);
         const float d = half_bits_to_float(
             *reinterpret_cast<const uint16_t*>(ring + (sb % G::kRS) * kQ6aStage + brow * kQ6aRowB + off + 208));
         d24 = d * 16777216.0f;
         dm32 = -32.0f * d;
     };
     auto sc_read = [&](int cq, int sb) {
-        const int off = (2 * (sb0 + sb)) & 15;
+        const int off = block_off(sb);
         scb = *reinterpret_cast<const int8_t*>(ring + (sb % G::kRS) * kQ6aStage + brow * kQ6aRowB + off + 192 +
                                                4 * cq + ks);
     };
@@ -2208,13 +2228,13 @@ __device__ __forceinline__ void q6a_wg(const uint16_t* __restrict__ A, const uin
     }
 }
 
-template <bool ACC, int FMR>
+template <bool ACC, int FMR, bool ANY = false>
 __global__ __launch_bounds__(kQ6aThreads) void rf_gemm_q6k_f16a_kernel(const uint16_t* __restrict__ A,
                                                                         const uint8_t* __restrict__ W,
                                                                         float* __restrict__ D, int M, int N, int K,
                                                                         KSplit sp) {
     __shared__ __align__(16) uint8_t lds[Q6aGeom<FMR>::kLds];
-    q6a_wg<ACC, FMR>(A, W, D, M, N, K, xcd_remap((int)blockIdx.x, (int)gridDim.x), lds, sp);
+    q6a_wg<ACC, FMR, ANY>(A, W, D, M, N, K, xcd_remap((int)blockIdx.x, (int)gridDim.x), lds, sp);
 }
 
 // ── q4s: Q4_K GEMM on fp16 activations, 32 FMR x 64 tiles, K slices on waves
@@ -2962,7 +2982,7 @@ static hipError_t gemm_q4_f16(const uint16_t* A, const void* W, float* D, int M,
 constexpr int kQ6TallMinM = RF_Q6_TALL_MIN_M;
 constexpr int kQ6LeanMaxM = 64;      // 64-row tiles up to this M (at M = 128: 40.0 against 33.0 us)
 
-template <bool ACC, int FMR>
+template <bool ACC, int FMR, bool ANY>
 static void q6_f16_tiles(const uint16_t* A, const uint8_t* w, float* D, int M, int N, int K, hipStream_t st,
                          const PartBuf& part, const RowNorm* rn = nullptr) {
     const long tiles = (long)((M + 32 * FMR - 1) / (32 * FMR)) * (N / kQ6aBN);
@@ -2970,25 +2990,25 @@ static void q6_f16_tiles(const uint16_t* A, const uint8_t* w, float* D, int M, i
     const int S = 2 * tiles <= (long)per_cu * device_cu_count() ? ksplit_count(tiles, K / kQK, M, N, part, per_cu)
                                                                   : 1;
     if (S > 1) {
-        hipLaunchKernelGGL((rf_gemm_q6k_f16a_kernel<false, FMR>), dim3((unsigned)(tiles * S)), dim3(kQ6aThreads), 0,
-                           st, A, w, nullptr, M, N, K, KSplit{S, part.p});
+        hipLaunchKernelGGL((rf_gemm_q6k_f16a_kernel<false, FMR, ANY>), dim3((unsigned)(tiles * S)), dim3(kQ6aThreads),
+                           0, st, A, w, nullptr, M, N, K, KSplit{S, part.p});
         reduce_for(ACC, nullptr, part.p, S, M, N, D, st, rn);
     } else {
-        hipLaunchKernelGGL((rf_gemm_q6k_f16a_kernel<ACC, FMR>), dim3((unsigned)tiles), dim3(kQ6aThreads), 0, st, A, w,
-                           D, M, N, K, KSplit{1, nullptr});
+        hipLaunchKernelGGL((rf_gemm_q6k_f16a_kernel<ACC, FMR, ANY>), dim3((unsigned)tiles), dim3(kQ6aThreads), 0, st,
+                           A, w, D, M, N, K, KSplit{1, nullptr});
     }
 }
 
-template <bool ACC>
+template <bool ACC, bool ANY = false>
 static hipError_t gemm_q6_f16(const uint16_t* A, const void* W, float* D, int M, int N, int K, hipStream_t st,
                               const PartBuf& part, const RowNorm* rn = nullptr) {
     const uint8_t* w = static_cast<const uint8_t*>(W);
     if (M >= kQ6TallMinM)
-        q6_f16_tiles<ACC, 8>(A, w, D, M, N, K, st, part, rn);
+        q6_f16_tiles<ACC, 8, ANY>(A, w, D, M, N, K, st, part, rn);
     else if (M <= kQ6LeanMaxM)
-        q6_f16_tiles<ACC, 2>(A, w, D, M, N, K, st, part, rn);
+        q6_f16_tiles<ACC, 2, ANY>(A, w, D, M, N, K, st, part, rn);
     else
-        q6_f16_tiles<ACC, 4>(A, w, D, M, N, K, st, part, rn);
+        q6_f16_tiles<ACC, 4, ANY>(A, w, D, M, N, K, st, part, rn);
     return hipGetLastError();
 }
 
@@ -3085,10 +3105,19 @@ extern "C" hipError_t wmma_gemm_q6_k_launch(const float* input, const void* weig
     if ((M % 64) != 0 || (N % 64) != 0 || (K % kQK) != 0) return hipErrorInvalidValue;
     if (!aligned16(input) || (reinterpret_cast<uintptr_t>(weights_q6_k) & 1u)) return hipErrorInvalidValue;
     GemmSlot slot;
-    // the fp16 tiles read 16-byte aligned weight rows (K % 2048)
-    if (K % 2048 == 0 && aligned16(weights_q6_k) && staging_slot(stream, K, &slot))
+    // the fp16 tiles, rows on 16-byte pieces (K % 2048 == 0) or anywhere (ANY;
+    // their split reduction stores float4, the fp32 tiles take any output).
+    // From three super-blocks on: below, the conversion pass costs what the
+    // tiles save.  Us on MI355X, fp32 tiles against these: 64 x 192 x 256
+    // 8.6 / 10.3, 256 x 192 x 512 14.6 / 16.3, 64 x 192 x 768 21.1 / 13.6,
+    // 512 x 1024 x 768 21.7 / 19.9, 512 x 1024 x 3584 149 / 27.5,
+    // 128 x 5120 x 13824 529 / 48, 512 x 3584 x 18944 737 / 125.
+    const bool any = K % 2048 != 0;
+    if (aligned16(weights_q6_k) && (!any || (K >= 3 * kQK && aligned16(output))) && staging_slot(stream, K, &slot))
         return staged_rows(input, M, K, slot, stream, [&](const uint16_t* a16, int m0, int rows, const PartBuf& pb) {
-            return gemm_q6_f16<false>(a16, weights_q6_k, output + (size_t)m0 * N, rows, N, K, stream, pb);
+            float* d = output + (size_t)m0 * N;
+            return any ? gemm_q6_f16<false, true>(a16, weights_q6_k, d, rows, N, K, stream, pb)
+                       : gemm_q6_f16<false>(a16, weights_q6_k, d, rows, N, K, stream, pb);
         });
     return launch_gemm<true>(input, weights_q6_k, output, M, N, K, stream, single_seg(N));
 }
