@@ -14,11 +14,15 @@
 //    matrix.  K split across the waves of a workgroup (8 super-blocks per
 //    wave), x held in registers, weights read with lane-linear aligned
 //    16-byte loads and restaged per wave through LDS.
-//  * rf_q6k_gemv_xreg_kernel: K <= 16384 otherwise.  Same K split and x
-//    registers, each lane loading its block fields directly (16-byte loads
-//    at the 2-byte aligned block offsets).
-//  * rf_q6k_gemv_kernel: larger K.  One row per wave step, four lanes per
+//  * rf_q6k_gemv_any_kernel: K <= 32768 otherwise, 16-byte aligned matrix.
+//    The same, with rows that start anywhere in a 16-byte piece.
+//  * rf_q6k_gemv_xreg_kernel: K <= 16384, matrices off a 16-byte address.
+//    Same K split and x registers, each lane loading its block fields
+//    directly (16-byte loads at the 2-byte aligned block offsets).
+//  * rf_q6k_gemv_kernel: the rest.  One row per wave step, four lanes per
 //    block, x in L2 (K*4 > 64 KB).
+#include <algorithm>
+
 #include "q6k_lin.h"
 
 
@@ -320,6 +324,25 @@ __global__ __launch_bounds__(512) void rf_q6k_gemv_lin_kernel(const uint8_t* __r
                     stage_lds + wave * 2048, part);
 }
 
+// The same for any K of up to MAXW slices (q6_lin_team's ANY form).  It reads
+// lane-linear pieces where rf_q6k_gemv_xreg_kernel's per-field loads at
+// 210-byte strides reach 2.3-2.7 TB/s.  us, before / after (MI355X, weights
+// beyond the Infinity Cache), same bits up to K = 16384: 152064 x 3584
+// 122 / 84, 151936 x 2560 113 / 80, 90178 x 5120 103 / 76, 5120 x 13824
+// 17.6 / 15.4, 4096 x 11008 13.4 / 11.8; above, where the row-step kernel was
+// bound by its x reads, 3584 x 18944 30.2 / 15.0, 8192 x 28672 94 / 39.
+template <int NB, int MAXW>
+__global__ __launch_bounds__(64 * MAXW) void rf_q6k_gemv_any_kernel(const uint8_t* __restrict__ w,
+                                                                    const float* __restrict__ x,
+                                                                    const float* residual, float* y, int K, int N,
+                                                                    int gk) {
+    __shared__ __align__(16) uint8_t stage_lds[MAXW * 2048];
+    extern __shared__ __align__(16) float part[];   // [rows of this workgroup][NWK][4 lane rows]
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    q6_lin_team<NB, true>(w, x, residual, y, K, N, nullptr, 1.0f, blockIdx.x, gridDim.x, wave, blockDim.x / kWave,
+                          stage_lds + wave * 2048, part, gk);
+}
+
 }  // namespace rf
 
 using namespace rf;
@@ -338,6 +361,30 @@ static hipError_t launch_q6(const void* weights_q6_k, const float* input, const 
         if (lds <= 64 * 1024) {
             hipLaunchKernelGGL((rf_q6k_gemv_lin_kernel<kQ6Ring>), dim3(grid), dim3(nwk * 64), lds, stream, w, input,
                                residual, output, n_rows, ncols_dst, nullptr, 0.0f);
+            return hipGetLastError();
+        }
+    }
+    // below a megabyte the launch is a row or two a wave and its latency counts:
+    // the direct loads are quicker (512 x 1280 2.84 against 3.01 us, 129 x 1792
+    // 2.6 against 2.8; 1001 x 2304, 1.9 MB, 4.29 against 3.88)
+    if (nsb <= 128 && (reinterpret_cast<uintptr_t>(w) & 15u) == 0 &&
+        (nsb > 64 || (size_t)ncols_dst * nsb * kQ6KBytes >= (1u << 20))) {
+        const int nwk = (nsb + 7) / 8;
+        // a multiple of 8, so that the rows of a workgroup share their phase;
+        // with two to seven slices twice the workgroups are faster (151936 x 2560
+        // 80 against 89 us, 4096 x 11008 11.8 against 12.3; one slice 121971 x
+        // 1536 45 against 39, ten 3584 x 18944 17.2 against 15.0)
+        const int cap = std::max(device_cu_count() * (nwk >= 4 ? 1 : 8 / nwk) / 8 * 8, 8);
+        const int gk = ncols_dst > cap && nwk >= 2 && nwk <= 7 ? 2 : 1;
+        const int grid = ncols_dst < cap ? ncols_dst : cap * gk;
+        const size_t lds = (size_t)((ncols_dst + grid - 1) / grid) * nwk * 4 * sizeof(float);
+        if (lds + (nwk <= 8 ? 8 : 16) * 2048 <= 64 * 1024) {
+            if (nwk <= 8)
+                hipLaunchKernelGGL((rf_q6k_gemv_any_kernel<kQ6Ring, 8>), dim3(grid), dim3(nwk * 64), lds, stream, w,
+                                   input, residual, output, n_rows, ncols_dst, gk);
+            else
+                hipLaunchKernelGGL((rf_q6k_gemv_any_kernel<kQ6Ring, 16>), dim3(grid), dim3(nwk * 64), lds, stream, w,
+                                   input, residual, output, n_rows, ncols_dst, gk);
             return hipGetLastError();
         }
     }

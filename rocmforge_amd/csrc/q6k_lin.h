@@ -76,6 +76,19 @@ __device__ __forceinline__ void q6_x_prep(float (&xr)[2][16], float (&xs)[2]) {
 // ~7.7 TB/s against ~4 TB/s with per-lane 16-byte loads at 2-byte aligned
 // block offsets.
 //
+// ANY: K any multiple of 256 (the last wave takes the row's remaining
+// super-blocks, its other lanes idle) and rows starting anywhere in a 16-byte
+// piece.  A wave's part is read as the 16-byte aligned window around it, whose
+// phase is one for all the rows of a workgroup: G is a multiple of 8 or there
+// is one row, and 8 rows are a multiple of 16 bytes.  The matrix is 16-byte
+// aligned, so only its last piece can reach past its end: that one is read at
+// the matrix's last 16 bytes and shifted into place.  Row sums are then
+// grouped per wave, ((r0 + r1) + (r2 + r3)) in team-wave order, and which of a
+// lane's two products is rounded before the fma follows the row's place in the
+// ring: the bits that rf_q6k_gemv_xreg_kernel, which takes any 2-byte aligned
+// matrix, compiles to (a decode step's 8-bit inputs turn a last-bit change into
+// one of 1e-3, so a layer's kernels keep theirs).
+//
 // Row j's sum is the team's 4 nwk partial sums (16-lane row sums, in
 // team-wave order) added in that order, whatever the grid.  Every thread of
 // the workgroup calls this once (one barrier before the final sums); part
@@ -83,17 +96,30 @@ __device__ __forceinline__ void q6_x_prep(float (&xr)[2][16], float (&xs)[2]) {
 struct Q6Seg {
     u32x4 a, b;
 };
+typedef uint32_t u32x4a2 __attribute__((ext_vector_type(4), aligned(2)));
 
-template <int NB>
+// v shifted down by `bytes` (even, 0..14, the same in all lanes)
+__device__ __forceinline__ u32x4 shift_down(u32x4 v, int bytes) {
+    if (bytes & 8) v = u32x4{v.z, v.w, 0u, 0u};
+    if (bytes & 4) v = u32x4{v.y, v.z, v.w, 0u};
+    if (bytes & 2)
+        v = u32x4{__builtin_amdgcn_alignbit(v.y, v.x, 16), __builtin_amdgcn_alignbit(v.z, v.y, 16),
+                  __builtin_amdgcn_alignbit(v.w, v.z, 16), v.w >> 16};
+    return v;
+}
+
+template <int NB, bool ANY = false>
 __device__ __forceinline__ void q6_lin_team(const uint8_t* __restrict__ w, const float* __restrict__ x,
                                             const float* residual, float* y, int K, int N,
                                             const float* __restrict__ norm_w, float inv, int g, int G, int tw,
-                                            int nwk, uint8_t* stage, float* part) {
+                                            int nwk, uint8_t* stage, float* part, int gk = 1) {
     const int lane = threadIdx.x & (kWave - 1);
     const int nsb = K / kQK;
     const size_t row_bytes = (size_t)nsb * kQ6KBytes;
     const int blk = lane >> 3;
-    const int sb = 8 * tw + blk;
+    const int nblk = ANY ? min(8, nsb - 8 * tw) : 8;
+    const bool live = blk < nblk;
+    const int sb = ANY && !live ? nsb - 1 : 8 * tw + blk;
     const int p = lane & 7;
     const int n = p >> 2;
     const int hq = (p & 3) >> 1;
@@ -117,9 +143,29 @@ __device__ __forceinline__ void q6_lin_team(const uint8_t* __restrict__ w, const
     }
     float xs[2];
     const uint8_t* wseg = w + (size_t)(8 * tw) * kQ6KBytes;
-    const int c1 = min(64 + lane, 104);   // chunks 105..127 re-read chunk 104 (same line), written to the spare area
+    const int phase = ANY ? (int)(((size_t)(g < N ? g : 0) * row_bytes + (size_t)(8 * tw) * kQ6KBytes) & 15) : 0;
+    const int last = ANY ? (phase + nblk * kQ6KBytes + 15) / 16 - 1 : 104;
+    // chunks past the last re-read it (same line), written to the spare area
+    const int c0 = ANY ? min(lane, last) : lane, c1 = min(64 + lane, last);
+    const int over = ANY ? (int)(0u - (uint32_t)((size_t)N * row_bytes)) & 15 : 0;   // of the matrix's last piece
+    // row j is row j0 + gk j of the G / gk workgroups the association refers to,
+    // of whose nr0 rows the first ring_rows are in the pipeline's full rounds
+    const int g0 = ANY ? G / gk : 1, j0 = ANY ? g / g0 : 0;
+    const int nr0 = g < N ? (N - 1 - (g - j0 * g0)) / g0 + 1 : 0;
+    const int ring_rows = nr0 < NB ? 0 : nr0 / NB * NB;
+    const bool tail = ANY && over && 8 * tw + nblk == nsb;
     auto load = [&](Q6Seg& u, int j) {
-        const uint8_t* src = wseg + (size_t)(nrows ? g + min(j, nrows - 1) * G : 0) * row_bytes;
+        const int row = nrows ? g + min(j, nrows - 1) * G : 0;
+        const uint8_t* src = wseg + (size_t)row * row_bytes;
+        if constexpr (ANY) {
+            src -= phase;
+            const int back = tail && row == N - 1 ? over : 0;
+            u.a = __builtin_nontemporal_load(
+                reinterpret_cast<const u32x4a2*>(src + 16 * c0 - (c0 == last ? back : 0)));
+            u.b = __builtin_nontemporal_load(
+                reinterpret_cast<const u32x4a2*>(src + 16 * c1 - (c1 == last ? back : 0)));
+            return;
+        }
         // nontemporal: each byte is read once; measured 6 % faster than
         // plain loads for the 4096 x 14336 ffn_down (no line is shared
         // between load instructions here, unlike the Q4_K unit loads)
@@ -132,7 +178,7 @@ __device__ __forceinline__ void q6_lin_team(const uint8_t* __restrict__ w, const
     // each scale byte / d as the aligned dword holding it.  (Unaligned
     // 16-byte LDS reads at these offsets measured ~4 us slower per launch.)
     const uint32_t* st32 = reinterpret_cast<const uint32_t*>(stage);
-    const int blkoff = blk * kQ6KBytes;
+    const int blkoff = phase + blk * kQ6KBytes;
     const uint32_t sh = 8u * (uint32_t)(blkoff & 3);
     const int qlw = (blkoff + 16 * p) >> 2;
     const int qhw = (blkoff + 128 + 32 * n + 16 * is) >> 2;
@@ -149,8 +195,13 @@ __device__ __forceinline__ void q6_lin_team(const uint8_t* __restrict__ w, const
                      __builtin_amdgcn_alignbit(d[3], d[2], s), __builtin_amdgcn_alignbit(d[4], d[3], s)};
     };
     auto process = [&](const Q6Seg& u, int j) {
-        *reinterpret_cast<u32x4*>(stage + 16 * lane) = u.a;
-        *reinterpret_cast<u32x4*>(stage + 16 * (64 + lane)) = u.b;
+        u32x4 ua = u.a, ub = u.b;
+        if (ANY && tail && g + j * G == N - 1) {
+            if (c0 == last) ua = shift_down(ua, over);
+            if (c1 == last) ub = shift_down(ub, over);
+        }
+        *reinterpret_cast<u32x4*>(stage + 16 * lane) = ua;
+        *reinterpret_cast<u32x4*>(stage + 16 * (64 + lane)) = ub;
         const u32x4 ql = field(qlw, sh);
         // qh shifted right by a further 2 hq bits in the same funnel shift:
         // only bits 0-1 and 4-5 of each byte are used below, so the bits
@@ -172,19 +223,35 @@ __device__ __forceinline__ void q6_lin_team(const uint8_t* __restrict__ w, const
         }
         float t0, t1;
         q6_dot16x2(v0, xr[0], v1, xr[1], t0, t1);
-        float acc = s0 * (t0 - 32.0f * xs[0]);
-        acc += s1 * (t1 - 32.0f * xs[1]);
+        float acc;
+        if constexpr (ANY) {
+            const float u0 = t0 - 32.0f * xs[0], u1 = t1 - 32.0f * xs[1];
+            const float f0 = __builtin_fmaf(s0, u0, __fmul_rn(s1, u1)), f1 = __builtin_fmaf(s1, u1, __fmul_rn(s0, u0));
+            const int jr = j0 + gk * j;
+            acc = jr % NB != 0 && jr < ring_rows ? f0 : f1;
+        } else {
+            acc = s0 * (t0 - 32.0f * xs[0]);
+            acc += s1 * (t1 - 32.0f * xs[1]);
+        }
         // the four 16-lane row sums go to LDS (no cross-row broadcast and
         // no read-lane per row); the final pass adds them in fixed order
-        const float r16 = row16_sum(acc);
-        if ((lane & 15) == 0) part[(j * nwk + tw) * 4 + (lane >> 4)] = r16;
+        const float r16 = row16_sum(ANY && !live ? 0.0f : acc);
+        // (a row's lanes add their quads in rotated orders; ANY keeps lane 15's,
+        // the one a full wave sum passes on)
+        if ((lane & 15) == (ANY ? 15 : 0)) part[(j * nwk + tw) * 4 + (lane >> 4)] = r16;
     };
     Q6Seg ring[NB];
     ring_pipeline<NB>(nrows, ring, load, process, [&]() { q6_x_prep(xr, xs); });
     __syncthreads();
     for (int j = tw * kWave + lane; j < nrows; j += nwk * kWave) {
         float t = 0.0f;
-        for (int k = 0; k < 4 * nwk; ++k) t += part[j * nwk * 4 + k];
+        if constexpr (ANY)
+            for (int k = 0; k < nwk; ++k) {
+                const float* q = part + (j * nwk + k) * 4;
+                t += (q[0] + q[1]) + (q[2] + q[3]);
+            }
+        else
+            for (int k = 0; k < 4 * nwk; ++k) t += part[j * nwk * 4 + k];
         y[g + j * G] = t + (residual ? residual[g + j * G] : 0.0f);
     }
 }

@@ -1,0 +1,44 @@
+"""Q6_K GEMV with rows that start anywhere in a 16-byte piece, at the edges of
+the K-split kernel's range, against the oracle's float64 evaluation."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import oracle as O
+from rocmforge_amd import synth
+
+from . import gpu_util as G
+
+pytestmark = pytest.mark.gpu
+
+
+# one slice and part of one, one block past a slice, the last slice full but
+# for one block; K = 16384 + 256 (nine slices) and 32768 (sixteen), 33024 beyond;
+# one row a workgroup, one more than that (ragged last rows), odd N (the
+# matrix ends inside a 16-byte piece) and N % 8 == 0 (it ends on one)
+@pytest.mark.parametrize("k,n", [(256, 5001), (1792, 1001), (2304, 1001), (2560, 2056), (3840, 4099), (5120, 600),
+                                 (11008, 257), (16128, 640), (16640, 5), (16640, 301), (18944, 513), (32768, 264),
+                                 (33024, 31)])
+def test_any_k_against_the_oracle(rf, dev, k, n):
+    w, x = synth.weights("q6_k", n, k, seed=k + n), synth.activations(k, seed=k)
+    res = np.random.default_rng(n).standard_normal(n).astype(np.float32)
+    dw, dx, dr = G.to_dev(w), G.to_dev(x), G.to_dev(res)
+    y, yr = G.empty(n, torch.float32), G.empty(n, torch.float32)
+    G.call(rf.gemv_q6_k_f32_launch, G.ptr(dw), G.ptr(dx), G.ptr(y), k, n)
+    G.call(rf.gemv_q6_k_f32_residual_launch, G.ptr(dw), G.ptr(dx), G.ptr(dr), G.ptr(yr), k, n)
+    ref = O.gemv_q6k(w, x, k, n)
+    rel, worst = G.gemv_error(G.host(y), ref)
+    assert rel <= 1e-5 and worst <= 1.0, (rel, worst)
+    np.testing.assert_array_equal(G.host(yr), G.host(y) + res)
+
+
+@pytest.mark.parametrize("k,n", [(2560, 4099), (3584, 1025), (11008, 1100), (1280, 5000)])
+def test_same_bits_as_a_matrix_off_a_16_byte_address(rf, dev, k, n):
+    # which the kernel with direct loads takes
+    w, x = synth.weights("q6_k", n, k, seed=k + 1), synth.activations(k, seed=k + 2)
+    raw = G.to_dev(np.concatenate([np.zeros(2, np.uint8), w.reshape(-1)]))
+    dw, dx = G.to_dev(w), G.to_dev(x)
+    a, b = G.empty(n, torch.float32), G.empty(n, torch.float32)
+    G.call(rf.gemv_q6_k_f32_launch, G.ptr(dw), G.ptr(dx), G.ptr(a), k, n)
+    G.call(rf.gemv_q6_k_f32_launch, G.ptr(raw[2:]), G.ptr(dx), G.ptr(b), k, n)
+    np.testing.assert_array_equal(G.host(a), G.host(b))
