@@ -11,7 +11,7 @@
 // accumulate / SwiGLU launchers below) round A to fp16 in a pass of their
 // own into library-owned device memory (the same values the reference's
 // __float2half gives) and run the fp16-activation tiles:
-//  * rf_gemm_q4k_f16a_kernel (Q4_K where 256 x 128 tiles fill at least 3/4
+//  * rf_gemm_q4k_f16a_kernel (Q4_K where 256 x 128 tiles fill more than half
 //    of the CUs): 4 waves, each weight dequantised once per 256 rows of A,
 //    A and the weight ring by LDS DMA.
 //  * rf_gemm_q4k_f16s_kernel (Q4_K otherwise) and rf_gemm_q6k_f16a_kernel
@@ -1480,15 +1480,15 @@ struct KSplit {
 // store silu(gate) * up into D[M x N] (N = the gate/up row count) as fp32
 // (PAIR 1) or rounded to fp16 (PAIR 2, D read as halves).  PAIR 3: a plain
 // tile whose store is the up projection of a SwiGLU, fp16 silu(G) * sum
-// with the gate product G [M x N] read back.  sp: K split (plain tiles,
-// PAIR_ARG 0, only).
+// with the gate product G [M x N] read back.  PAIR 4: a plain tile added to
+// D's old contents.  sp: K split (plain tiles, PAIR_ARG 0, only).
 template <int PAIR_ARG>
 __global__ __launch_bounds__(kF16aThreads) void rf_gemm_q4k_f16a_kernel(const uint16_t* __restrict__ A,
                                                                          const uint8_t* __restrict__ W,
                                                                          const uint8_t* __restrict__ W1,
                                                                          float* __restrict__ D, int M, int N, int K,
                                                                          const float* __restrict__ G, KSplit sp) {
-    constexpr int PAIR = PAIR_ARG == 3 ? 0 : PAIR_ARG;      // 3: a plain tile, gated store
+    constexpr int PAIR = PAIR_ARG >= 3 ? 0 : PAIR_ARG;      // 3, 4: a plain tile, gated / accumulating store
     // one LDS block: ring (2 stages), A (3 buffers), scale tables (2); after
     // the loop its first 128 KB carry the K-half exchange
     __shared__ __align__(16) uint8_t lds[kF16aLds];
@@ -1739,7 +1739,21 @@ __global__ __launch_bounds__(kF16aThreads) void rf_gemm_q4k_f16a_kernel(const ui
         constexpr int keep = KH ? 4 : 0;
         const int partner = wave ^ 1;
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < 4; ++i) {
+            // the old contents of a row block, all in flight before its first store
+            float old[2][4][4];
+            if constexpr (PAIR_ARG == 4) {
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+#pragma unroll
+                    for (int q = 0; q < 4; ++q)
+#pragma unroll
+                        for (int u = 0; u < 4; ++u) {
+                            const int row = m0 + 32 * (keep + i) + 8 * q + 4 * h + u;
+                            old[j][q][u] = D[(size_t)(FULL ? row : min(row, M - 1)) * N + n0 + 64 * wn + 32 * j + col];
+                        }
+                __builtin_amdgcn_sched_barrier(0);
+            }
 #pragma unroll
             for (int j = 0; j < 2; ++j) {
                 const int ncol = n0 + 64 * wn + 32 * j + col;
@@ -1758,12 +1772,15 @@ __global__ __launch_bounds__(kF16aThreads) void rf_gemm_q4k_f16a_kernel(const ui
                         if constexpr (PAIR_ARG == 3) {      // up projection of a SwiGLU: fp16 silu(gate) * up
                             const float gg = G[e];
                             reinterpret_cast<uint16_t*>(D)[e] = f16_bits_rn(gg / (1.0f + expf(-gg)) * sum);
+                        } else if constexpr (PAIR_ARG == 4) {
+                            D[e] = old[j][q][u] + sum;
                         } else {
                             D[e] = sum;
                         }
                     }
                 }
             }
+        }
     };
     if (kh)
         give_half(std::integral_constant<int, 1>{});
@@ -2886,7 +2903,7 @@ static void reduce_for(bool acc, const float* G, const float* part, int S, int M
 }
 
 // Q4_K on fp16 activations: 256 x 128 tiles (rf_gemm_q4k_f16a_kernel) where
-// they fill at least three quarters of the CUs, else the eight-wave
+// they fill more than half the CUs, else the eight-wave
 // K-sliced tiles (rf_gemm_q4k_f16s_kernel) of 256 rows (from M =
 // kQ4TallMinM: each weight dequantised once per 256 rows), 64 rows (M <= 64,
 // or when they come to at most one round of CUs) or 128, split over K when
@@ -2921,8 +2938,17 @@ static hipError_t gemm_q4_f16(const uint16_t* A, const void* W, float* D, int M,
                               const float* G, const PartBuf& part, const RowNorm* rn = nullptr) {
     const uint8_t* w = static_cast<const uint8_t*>(W);
     const long big = (long)((M + kF16aBM - 1) / kF16aBM) * (N % kF16aBN == 0 ? N / kF16aBN : 0);
-    if (!ACC && 4 * big >= 3L * device_cu_count()) {
-        if (G != nullptr)
+    // From half the CUs: there twice as many 256 x 64 tiles need a second round,
+    // each costing 2/3 of a 256 x 128 tile's (us, 256 x 64 against 256 x 128 fp16
+    // A on MI355X: 512 x 9216 x 4096, 144 tiles, 78 / 62; 1984 x 2560 x 9728,
+    // 160, 164 / 123; 1280 x 3840 x 2560, 150, 54 / 38; 1088 x 3584 x 18944,
+    // 140, 280 / 209).  Accumulating (the old contents of a row block read ahead
+    // of its stores) 2048 x 4096 x 12288 263 / 215, 2048 x 4096 x 4096 101 / 76.
+    if (2 * big > (long)device_cu_count()) {
+        if constexpr (ACC)
+            hipLaunchKernelGGL(rf_gemm_q4k_f16a_kernel<4>, dim3((unsigned)big), dim3(kF16aThreads), 0, st, A, w, w, D,
+                               M, N, K, nullptr, KSplit{1, nullptr});
+        else if (G != nullptr)
             hipLaunchKernelGGL(rf_gemm_q4k_f16a_kernel<3>, dim3((unsigned)big), dim3(kF16aThreads), 0, st, A, w, w, D,
                                M, N, K, G, KSplit{1, nullptr});
         else
