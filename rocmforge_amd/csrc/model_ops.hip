@@ -42,16 +42,11 @@ namespace rf {
 constexpr float kNegMax = -3.402823466e+38f;
 
 __device__ __forceinline__ float wave_max(float v) {
-    // butterfly over the 64 lanes: every lane ends with the maximum
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o));
-    return v;
+    return xor_max<32, 1>(v);   // every lane ends with the maximum
 }
 
 __device__ __forceinline__ float wave_sum_all(float v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-    return v;
+    return xor_sum64(v);
 }
 
 // theta_i = 1 / base^((float)(2i) / (float)d), evaluated in double and
@@ -359,8 +354,7 @@ __device__ __forceinline__ void head_norm_rope(float v[8], int sub, bool norm, c
         float ss = v[0] * v[0];
 #pragma unroll
         for (int i = 1; i < 8; ++i) ss = __fmaf_rn(v[i], v[i], ss);
-#pragma unroll
-        for (int o = 1; o < LPP; o <<= 1) ss += __shfl_xor(ss, o);
+        ss = xor_sum<1, LPP / 2>(ss);
         const float inv = rsqrtf(ss / (float)D + eps);
 #pragma unroll
         for (int i = 0; i < 8; ++i) v[i] = (v[i] * inv) * gv[i];
@@ -369,7 +363,7 @@ __device__ __forceinline__ void head_norm_rope(float v[8], int sub, bool norm, c
         const bool lo = sub < LPP / 2;
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
-            const float other = __shfl_xor(v[i], LPP / 2);
+            const float other = lane_xor<LPP / 2>(v[i]);
             float x0 = lo ? v[i] : other, x1 = lo ? other : v[i];
             rope_cs(x0, x1, c[i].x, c[i].y);
             v[i] = lo ? x0 : x1;
@@ -538,8 +532,7 @@ __global__ __launch_bounds__(256) void rf_attn_decode_kernel(float* __restrict__
                     s += qv[2 * t] * f.x + qv[2 * t + 1] * f.y;
                 }
             }
-#pragma unroll
-            for (int o = LPP / 2; o > 0; o >>= 1) s += __shfl_xor(s, o);
+            s = xor_sum<LPP / 2, 1>(s);
             if (p < cn && lane % LPP == 0) sc[p] = s * scale;
         }
         __syncthreads();
@@ -597,7 +590,9 @@ __global__ __launch_bounds__(256) void rf_attn_decode_kernel(float* __restrict__
 }
 
 // Split decode attention (the path used when the GQA group is at most 8
-// query heads).  Grid = (kv head, split); a workgroup has one wave per
+// query heads).  Bound: up to a few thousand positions the two launches and
+// one trip to memory; beyond, the K / V stream and the VALU beside it (each
+// position and head takes 256 FMAs, on fp16 operands at half rate).  Grid = (kv head, split); a workgroup has one wave per
 // query head of the kv head's group, so the group's K/V rows are read once
 // per workgroup (the other waves hit L1).  Positions go out in chunks of
 // kSplitChunk, chunk c to split c mod S, each wave keeping an online
@@ -608,6 +603,18 @@ __global__ __launch_bounds__(256) void rf_attn_decode_kernel(float* __restrict__
 // kernel merges the S partials of each head (rows of D + 4 floats: acc, m, l):
 //   out = sum_s e^(m_s - M) acc_s / sum_s e^(m_s - M) l_s,  M = max_s m_s.
 constexpr int kSplitChunk = 32;
+// Rounds of the splits (S chunks each) from which the sequence counts as long
+// and, at D = 128 with two query heads or more to a KV head, the chunks come
+// through an LDS ring (use_long): the walk over a chunk at a time waited for
+// each chunk's loads, read every row once per head and spent a third of its
+// VALU on exps that 16 lanes computed alike.  32 / 8 heads, both launches, us
+// before / after (caches beyond the Infinity Cache): 16200 positions
+// 31.5 / 23.4, 8192 (40 heads) 30.1 / 27.6, 32000 (64 heads) 85.5 / 55.8; at
+// 4096, two rounds, 14.1 / 14.5; with one head to a KV head the direct walk is
+// as fast (4500 positions 14.0 against 17.6).
+constexpr int kLongRounds = 3;
+constexpr int kLongStages = 4;
+constexpr int kLongHalf = kSplitChunk * 256;    // a chunk's K (or V) rows at D = 128
 
 // QK: the decode step's per-head Q/K norm, RoPE and KV write are folded in
 // (qk.*): q, k, v are the raw projections; every wave normalises and
@@ -641,10 +648,12 @@ __global__ __launch_bounds__(512) void rf_attn_split_kernel(const float* __restr
     constexpr int NI = kSplitChunk / PPW;       // load instructions per chunk (K and V each)
     __shared__ u32x4 new_kv[2][LPP];            // QK: the new position's fp16 K and V row of this kv head
     __shared__ __align__(16) float2 lcs[QK ? 8 : 1][QK ? D / 2 : 2];   // QK: each wave's cos / sin
+    __shared__ __align__(16) uint8_t ring[LPP == 16 ? kLongStages * 2 * kLongHalf : 16];
     const int seq = len_ptr ? *len_ptr : len0;
     const int kvh = blockIdx.x, split = blockIdx.y;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int head = kvh * (nh / nkv) + wave;
+    const int group = blockDim.x >> 6;      // nh / nkv
+    const int head = kvh * group + wave;
     const size_t row = (size_t)nkv * D;
     const int sub = lane % LPP, grp = lane / LPP;
     if (split * kSplitChunk >= seq) {       // no positions: an empty partial (l = 0) for the merge
@@ -655,8 +664,6 @@ __global__ __launch_bounds__(512) void rf_attn_split_kernel(const float* __restr
         }
         return;
     }
-    const __half* kh = kc + (size_t)kvh * D + 8 * sub;
-    const __half* vh = vc + (size_t)kvh * D + 8 * sub;
     const int pos = seq - 1;
     const bool owner = QK && split == (pos / kSplitChunk) % S;   // workgroup-uniform
     // loads in the order they are needed: q, (owner) the raw k / v, then the first chunk
@@ -676,98 +683,233 @@ __global__ __launch_bounds__(512) void rf_attn_split_kernel(const float* __restr
         load8(qk.v + (size_t)kvh * D + 8 * sub, vx);
         if (qk.k_norm != nullptr) load8(qk.k_norm + 8 * sub, gk);
     }
-    float m = kNegMax, l = 0.0f, acc[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) acc[j] = 0.0f;
-    for (int c0 = split * kSplitChunk; c0 < seq; c0 += S * kSplitChunk) {
-        u32x4 kk[NI], vv[NI];
+    // A chunk's rows; past the end of the sequence zeros
+    struct Rows {
+        u32x4 k[NI], v[NI];
+    };
+    auto load = [&](Rows& r, int c0) {
+        // (a pointer per lane: scalar bases with a lane offset cost 0.4 us a launch)
+        const __half* kh = kc + (size_t)kvh * D + 8 * sub;
+        const __half* vh = vc + (size_t)kvh * D + 8 * sub;
 #pragma unroll
         for (int i = 0; i < NI; ++i) {
             const int p = c0 + i * PPW + grp;
             const bool ok = p < seq;
-            kk[i] = ok ? *reinterpret_cast<const u32x4*>(kh + (size_t)p * row) : u32x4{0, 0, 0, 0};
-            vv[i] = ok ? *reinterpret_cast<const u32x4*>(vh + (size_t)p * row) : u32x4{0, 0, 0, 0};
+            r.k[i] = ok ? *reinterpret_cast<const u32x4*>(kh + (size_t)p * row) : u32x4{0, 0, 0, 0};
+            r.v[i] = ok ? *reinterpret_cast<const u32x4*>(vh + (size_t)p * row) : u32x4{0, 0, 0, 0};
         }
-        if constexpr (QK) {
-            if (c0 == split * kSplitChunk) {     // first chunk: the per-head step, while the loads fly
-                wave_cos_sin_put<LPP>(lcs[wave], csl, lane);
-                cs8<LPP>(lcs[wave], sub, qk.neox, cv);
-                head_norm_rope<LPP>(qv, sub, qk.q_norm != nullptr, gq, qk.eps, cv, qk.neox);
-                if (owner) {
-                    if (wave == 0) {
-                        head_norm_rope<LPP>(kx, sub, qk.k_norm != nullptr, gk, qk.eps, cv, qk.neox);
-                        if (grp == 0) {
-                            const size_t c = (size_t)pos * row + (size_t)kvh * D + 8 * sub;
-                            store8_f16(qk.kc + c, kx);
-                            store8_f16(qk.vc + c, vx);
-                            typedef _Float16 hv8 __attribute__((ext_vector_type(8)));
-                            hv8 hk, hvv;
+    };
+    float m = kNegMax, l = 0.0f, acc[8];
 #pragma unroll
-                            for (int i = 0; i < 8; ++i) {
-                                hk[i] = (_Float16)kx[i];
-                                hvv[i] = (_Float16)vx[i];
-                            }
-                            new_kv[0][sub] = __builtin_bit_cast(u32x4, hk);
-                            new_kv[1][sub] = __builtin_bit_cast(u32x4, hvv);
-                        }
-                    }
-                    __syncthreads();
-                }
-            }
+    for (int j = 0; j < 8; ++j) acc[j] = 0.0f;
+    // The roundings are spelled out, so that every instance of this code gives
+    // the same bits.
+    auto use = [&](Rows& r, int c0) {
+        if constexpr (QK) {
             if (owner && pos >= c0 && pos < c0 + kSplitChunk) {
                 // the row at pos was loaded before it was written: take it from LDS
 #pragma unroll
                 for (int i = 0; i < NI; ++i)
                     if (c0 + i * PPW + grp == pos) {
-                        kk[i] = new_kv[0][sub];
-                        vv[i] = new_kv[1][sub];
+                        r.k[i] = new_kv[0][sub];
+                        r.v[i] = new_kv[1][sub];
                     }
             }
         }
-        float sc[NI];
+        float tk[NI], sc[NI];
         float cm = kNegMax;
 #pragma unroll
         for (int i = 0; i < NI; ++i) {
-            const uint32_t w4[4] = {kk[i].x, kk[i].y, kk[i].z, kk[i].w};
+            const uint32_t w4[4] = {r.k[i].x, r.k[i].y, r.k[i].z, r.k[i].w};
             float t = 0.0f;
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
                 const float2 f = __half22float2(__builtin_bit_cast(__half2, w4[u]));
-                t += qv[2 * u] * f.x + qv[2 * u + 1] * f.y;
+                t = __fadd_rn(t, __fmaf_rn(qv[2 * u], f.x, __fmul_rn(qv[2 * u + 1], f.y)));
             }
-#pragma unroll
-            for (int o = LPP / 2; o > 0; o >>= 1) t += __shfl_xor(t, o);
-            sc[i] = (c0 + i * PPW + grp < seq) ? t * scale : kNegMax;
+            tk[i] = t = xor_sum<LPP / 2, 1>(t);
+            sc[i] = (c0 + i * PPW + grp < seq) ? __fmul_rn(t, scale) : kNegMax;
             cm = fmaxf(cm, sc[i]);
         }
-#pragma unroll
-        for (int o = LPP; o < 64; o <<= 1) cm = fmaxf(cm, __shfl_xor(cm, o));
+        cm = xor_max<LPP, 32>(cm);
         const float m_new = fmaxf(m, cm);
-        const float alpha = expf(m - m_new);
+        const float alpha = expf(__fsub_rn(m, m_new));
         float ls = 0.0f;
 #pragma unroll
-        for (int j = 0; j < 8; ++j) acc[j] *= alpha;
+        for (int j = 0; j < 8; ++j) acc[j] = __fmul_rn(acc[j], alpha);
 #pragma unroll
         for (int i = 0; i < NI; ++i) {
-            const float e = (c0 + i * PPW + grp < seq) ? expf(sc[i] - m_new) : 0.0f;
-            ls += e;
-            const uint32_t w4[4] = {vv[i].x, vv[i].y, vv[i].z, vv[i].w};
+            const float x = LPP == 16 ? __fmaf_rn(tk[i], scale, -m_new) : __fsub_rn(sc[i], m_new);
+            const float e = (c0 + i * PPW + grp < seq) ? expf(x) : 0.0f;
+            ls = __fadd_rn(ls, e);
+            const uint32_t w4[4] = {r.v[i].x, r.v[i].y, r.v[i].z, r.v[i].w};
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
                 const float2 f = __half22float2(__builtin_bit_cast(__half2, w4[u]));
-                acc[2 * u] += e * f.x;
-                acc[2 * u + 1] += e * f.y;
+                acc[2 * u] = __fmaf_rn(e, f.x, acc[2 * u]);
+                acc[2 * u + 1] = __fmaf_rn(e, f.y, acc[2 * u + 1]);
             }
         }
-#pragma unroll
-        for (int o = LPP; o < 64; o <<= 1) ls += __shfl_xor(ls, o);
-        l = l * alpha + ls;
+        ls = xor_sum<LPP, 32>(ls);
+        l = __fmaf_rn(l, alpha, ls);
         m = m_new;
+    };
+    // The same for long sequences (D = 128).  The 8 partial dots of a lane are
+    // added over the row's 16 lanes by a transposing butterfly, after which lane
+    // `sub` holds the score of load sub / 2 alone: one exp a lane instead of 8, its
+    // value handed back to the row by DPP broadcasts.  The maximum is reduced only
+    // when some score passes it, l stays a sum per lane (lanes 2 i, 2 i + 1 alike).
+    auto use_long = [&](const uint8_t* tile, int c0) {
+        Rows r;
+#pragma unroll
+        for (int i = 0; i < NI; ++i) {
+            r.k[i] = *reinterpret_cast<const u32x4*>(tile + 1024 * i + 16 * lane);
+            r.v[i] = *reinterpret_cast<const u32x4*>(tile + kLongHalf + 1024 * i + 16 * lane);
+        }
+        if (c0 + kSplitChunk >= seq) {
+            // rows past the end (copies of an earlier one) weigh nothing; the row at
+            // pos was loaded before it was written: take it from LDS
+#pragma unroll
+            for (int i = 0; i < NI; ++i) {
+                const int p = c0 + i * PPW + grp;
+                if (p >= seq) r.v[i] = u32x4{0, 0, 0, 0};
+                if (QK && p == pos) {
+                    r.k[i] = new_kv[0][sub];
+                    r.v[i] = new_kv[1][sub];
+                }
+            }
+        }
+        if constexpr (LPP == 16) {
+            typedef _Float16 h8r __attribute__((ext_vector_type(8)));
+            float t[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const h8r kh8 = __builtin_bit_cast(h8r, r.k[i]);
+                t[i] = 0.0f;
+#pragma unroll
+                for (int j = 0; j < 8; ++j) t[i] = __builtin_fmaf((float)kh8[j], qv[j], t[i]);
+            }
+            const bool b3 = sub & 8, b2 = sub & 4, b1 = sub & 2;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) t[i] = (b3 ? t[i + 4] : t[i]) + lane_xor<8>(b3 ? t[i] : t[i + 4]);
+#pragma unroll
+            for (int i = 0; i < 2; ++i) t[i] = (b2 ? t[i + 2] : t[i]) + lane_xor<4>(b2 ? t[i] : t[i + 2]);
+            t[0] = (b1 ? t[1] : t[0]) + lane_xor<2>(b1 ? t[0] : t[1]);
+            t[0] += lane_xor<1>(t[0]);
+            const bool in = c0 + (sub >> 1) * PPW + grp < seq;
+            const float s = in ? t[0] * scale : kNegMax;
+            if (__builtin_amdgcn_ballot_w64(s > m)) {
+                const float m_new = fmaxf(m, xor_max<2, 32>(s));
+                const float alpha = expf(m - m_new);
+                m = m_new;
+                l *= alpha;
+#pragma unroll
+                for (int j = 0; j < 8; ++j) acc[j] *= alpha;
+            }
+            const float e = in ? expf(s - m) : 0.0f;
+            l += e;
+            const float eb[8] = {dpp_f<0x150>(e), dpp_f<0x152>(e), dpp_f<0x154>(e), dpp_f<0x156>(e),   // row_newbcast
+                                 dpp_f<0x158>(e), dpp_f<0x15A>(e), dpp_f<0x15C>(e), dpp_f<0x15E>(e)};
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const h8r vh8 = __builtin_bit_cast(h8r, r.v[i]);
+#pragma unroll
+                for (int j = 0; j < 8; ++j) acc[j] = __builtin_fmaf((float)vh8[j], eb[i], acc[j]);
+            }
+        }
+    };
+    const int first_c = split * kSplitChunk, step = S * kSplitChunk;
+    const bool is_long = LPP == 16 && group > 1 && seq > kLongRounds * step;
+    // Long sequences: the chunks come through an LDS ring, loaded once a
+    // workgroup by LDS DMA kLongStages - 1 chunks ahead.  DMA instruction j of a
+    // chunk's 16 moves 4 rows of K (j < 8) or V; wave w issues j = w, w + group,
+    // .., the same number in every wave (repeating instruction 15).  Rows past
+    // the end re-read the last one (which the owner may be writing: what arrives
+    // for it and for them is not used).
+    int per_wave = 0, nch = 0;
+    const uint8_t* kb = reinterpret_cast<const uint8_t*>(kc) + (size_t)kvh * D * 2;      // wave-uniform
+    const uint8_t* vb = reinterpret_cast<const uint8_t*>(vc) + (size_t)kvh * D * 2;
+    const uint32_t loff = 2u * ((uint32_t)grp * (uint32_t)row + 8u * (uint32_t)sub);      // the lane's part
+    auto issue = [&](int t) {
+        const int c0 = first_c + min(t, nch - 1) * step;
+        const uint32_t dst = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)ring +
+                             (uint32_t)(t % kLongStages) * (2 * kLongHalf);
+        const size_t o = 2 * (size_t)c0 * row;
+        const int tail = seq - 1 - c0;
+        for (int i = 0; i < per_wave; ++i) {
+            const int j = __builtin_amdgcn_readfirstlane(min(wave + i * group, 15));
+            const uint8_t* base = (j < 8 ? kb : vb) + o;
+            const uint32_t d = __builtin_amdgcn_readfirstlane(dst + 1024u * (uint32_t)j);
+            if (tail >= kSplitChunk - 1)
+                lds_dma16(d, loff, base + (size_t)(8u * (uint32_t)(j & 7) * (uint32_t)row));
+            else
+                lds_dma16(d, 2u * (uint32_t)(min(4 * (j & 7) + grp, tail) * (int)row + 8 * sub), base);
+        }
+    };
+    // QK: the per-head step, while the first loads fly
+    auto per_head = [&]() {
+        if constexpr (QK) {
+            wave_cos_sin_put<LPP>(lcs[wave], csl, lane);
+            cs8<LPP>(lcs[wave], sub, qk.neox, cv);
+            head_norm_rope<LPP>(qv, sub, qk.q_norm != nullptr, gq, qk.eps, cv, qk.neox);
+            if (owner) {
+                if (wave == 0) {
+                    head_norm_rope<LPP>(kx, sub, qk.k_norm != nullptr, gk, qk.eps, cv, qk.neox);
+                    if (grp == 0) {
+                        const size_t c = (size_t)pos * row + (size_t)kvh * D + 8 * sub;
+                        store8_f16(qk.kc + c, kx);
+                        store8_f16(qk.vc + c, vx);
+                        typedef _Float16 hv8 __attribute__((ext_vector_type(8)));
+                        hv8 hk, hvv;
+    #pragma unroll
+                        for (int i = 0; i < 8; ++i) {
+                            hk[i] = (_Float16)kx[i];
+                            hvv[i] = (_Float16)vx[i];
+                        }
+                        new_kv[0][sub] = __builtin_bit_cast(u32x4, hk);
+                        new_kv[1][sub] = __builtin_bit_cast(u32x4, hvv);
+                    }
+                }
+                __syncthreads();
+            }
+        }
+    };
+    if (is_long) {
+        per_wave = (16 + group - 1) / group;
+        nch = ((seq + kSplitChunk - 1) / kSplitChunk - split + S - 1) / S;
+        for (int t = 0; t < kLongStages - 1; ++t) issue(t);
+        per_head();
+        for (int t = 0; t < nch; ++t) {
+            // chunk t has landed when the DMAs of the kLongStages - 2 chunks behind it
+            // are all that is in flight; past the barrier every wave's have, and the
+            // stage of chunk t - 1 has been read
+            switch (per_wave) {
+            case 2: asm volatile("s_waitcnt vmcnt(%0)" :: "n"(2 * (kLongStages - 2)) : "memory"); break;
+            case 3: asm volatile("s_waitcnt vmcnt(%0)" :: "n"(3 * (kLongStages - 2)) : "memory"); break;
+            case 4: asm volatile("s_waitcnt vmcnt(%0)" :: "n"(4 * (kLongStages - 2)) : "memory"); break;
+            case 6: asm volatile("s_waitcnt vmcnt(%0)" :: "n"(6 * (kLongStages - 2)) : "memory"); break;
+            case 8: asm volatile("s_waitcnt vmcnt(%0)" :: "n"(8 * (kLongStages - 2)) : "memory"); break;
+            case 16: asm volatile("s_waitcnt vmcnt(%0)" :: "n"(16 * (kLongStages - 2)) : "memory"); break;
+            default: asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            }
+            lds_barrier();
+            issue(t + kLongStages - 1);
+            use_long(ring + (t % kLongStages) * (2 * kLongHalf), first_c + t * step);
+        }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");     // no DMA outlives the workgroup's LDS
+        l = xor_sum<2, 32>(l);
+    } else {
+        // (one copy of each part: at these lengths the launch is short enough for
+        // its instruction fetches to show)
+        Rows r;
+        for (int c0 = first_c; c0 < seq; c0 += step) {
+            load(r, c0);
+            if (c0 == first_c) per_head();
+            use(r, c0);
+        }
     }
 #pragma unroll
-    for (int j = 0; j < 8; ++j)
-#pragma unroll
-        for (int o = LPP; o < 64; o <<= 1) acc[j] += __shfl_xor(acc[j], o);
+    for (int j = 0; j < 8; ++j) acc[j] = xor_sum<LPP, 32>(acc[j]);
     float* dst = ws + ((size_t)head * S + split) * (D + 4);
     if (grp == 0) {
         *reinterpret_cast<float4*>(dst + 8 * sub) = make_float4(acc[0], acc[1], acc[2], acc[3]);
@@ -830,13 +972,11 @@ __global__ __launch_bounds__(256) void rf_attn_merge_kernel(const float* __restr
     load(gr);                               // in flight with the (m, l) loads
     if (t < 64) {
         float M = mv;
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) M = fmaxf(M, __shfl_xor(M, o));
+        M = xor_max<32, 1>(M);
         const float f = lv > 0.0f ? expf(mv - M) : 0.0f;   // splits without positions count 0
         fs[t] = f;
         float lt = f * lv;
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) lt += __shfl_xor(lt, o);
+        lt = xor_sum64(lt);
         if (t == 0) lt_s = lt;
     }
     __syncthreads();
@@ -977,13 +1117,11 @@ __global__ __launch_bounds__(64 * kHeadWaves) void rf_attn_head_kernel(const flo
                 t = __fmaf_rn(qv[2 * u], f.x, t);
                 t = __fmaf_rn(qv[2 * u + 1], f.y, t);
             }
-#pragma unroll
-            for (int o = LPP / 2; o > 0; o >>= 1) t += __shfl_xor(t, o);
+            t = xor_sum<LPP / 2, 1>(t);
             sc[i] = ((b0 + kHeadWaves * i) * PPW + grp < seq) ? __fmul_rn(t, scale) : kNegMax;
             cm = fmaxf(cm, sc[i]);
         }
-#pragma unroll
-        for (int o = LPP; o < 64; o <<= 1) cm = fmaxf(cm, __shfl_xor(cm, o));
+        cm = xor_max<LPP, 32>(cm);
         const float m_new = fmaxf(m, cm);
         const float alpha = expf(m - m_new);
         float ls = 0.0f;
@@ -1001,8 +1139,7 @@ __global__ __launch_bounds__(64 * kHeadWaves) void rf_attn_head_kernel(const flo
                 acc[2 * u + 1] = __fmaf_rn(e, f.y, acc[2 * u + 1]);
             }
         }
-#pragma unroll
-        for (int o = LPP; o < 64; o <<= 1) ls += __shfl_xor(ls, o);
+        ls = xor_sum<LPP, 32>(ls);
         l = __fmaf_rn(l, alpha, ls);
         m = m_new;
     }
@@ -1010,8 +1147,7 @@ __global__ __launch_bounds__(64 * kHeadWaves) void rf_attn_head_kernel(const flo
     // above ran; waves without positions leave m = kNegMax, l = 0)
 #pragma unroll
     for (int j = 0; j < 8; ++j)
-#pragma unroll
-        for (int o = LPP; o < 64; o <<= 1) acc[j] += __shfl_xor(acc[j], o);
+        acc[j] = xor_sum<LPP, 32>(acc[j]);
     if (grp == 0) {
         *reinterpret_cast<float4*>(&wacc[wave][8 * sub]) = make_float4(acc[0], acc[1], acc[2], acc[3]);
         *reinterpret_cast<float4*>(&wacc[wave][8 * sub + 4]) = make_float4(acc[4], acc[5], acc[6], acc[7]);
@@ -1881,7 +2017,7 @@ void rf_attn_prefill_kernel(const _Float16* __restrict__ Q, const _Float16* __re
         for (int b = 0; b < 2; ++b)
 #pragma unroll
             for (int e = 0; e < 16; ++e) tmax = fmaxf(tmax, s[b][e]);
-        tmax = fmaxf(tmax, __shfl_xor(tmax, 32)) * scale2;
+        tmax = fmaxf(tmax, lane_xor<32>(tmax)) * scale2;
         // O is rescaled only where some lane's maximum moved.  (A maximum left behind
         // by up to 2^8 saves 6 % of the time, but then a row's largest weight is no
         // longer exactly one and peaked rows lose half their precision.)
@@ -1942,7 +2078,7 @@ void rf_attn_prefill_kernel(const _Float16* __restrict__ Q, const _Float16* __re
         if (ks > 0) return;
     }
     if (!active) return;
-    l += __shfl_xor(l, 32);                      // each half wave summed its own keys
+    l += lane_xor<32>(l);                      // each half wave summed its own keys
     const float inv_l = l > 0.0f ? 1.0f / l : 0.0f;
     OUT* orow = O + (size_t)query * qrow + (size_t)head * kAttD;
 #pragma unroll

@@ -162,26 +162,53 @@ __device__ __forceinline__ float sq8(const float4& a, const float4& b) {
     return t;
 }
 
-// The xor butterfly v += v[lane ^ o], o = 32, 16, .., 1, every lane ending
-// with the same sum, on VALU exchanges: v_permlane32_swap / _16_swap for 32
-// and 16, DPP row_ror:8 for 8, row_shl:4 / row_shr:4 selected by lane bit 2
-// for 4, quad permutes for 2 and 1 -- the sums of the __shfl_xor form bit for
-// bit (each step adds the same partner), without its LDS round trips.
-__device__ __forceinline__ float xor_sum64(float v) {
+// v of lane ^ O (O = 1, 2, .., 32) by VALU exchanges, without the LDS round
+// trip of __shfl_xor: v_permlane32_swap / _16_swap for 32 and 16, DPP
+// row_ror:8 for 8, row_shl:4 / row_shr:4 selected by lane bit 2 for 4, quad
+// permutes for 2 and 1.
+template <int O>
+__device__ __forceinline__ float lane_xor(float v) {
+    static_assert(O == 1 || O == 2 || O == 4 || O == 8 || O == 16 || O == 32, "one lane bit");
     const int lane = threadIdx.x & 63;
-    const uint32_t b32 = __float_as_uint(v);
-    const auto r32 = __builtin_amdgcn_permlane32_swap(b32, b32, false, false);
-    v += __uint_as_float(lane >= 32 ? r32[0] : r32[1]);
-    const uint32_t b16 = __float_as_uint(v);
-    const auto r16 = __builtin_amdgcn_permlane16_swap(b16, b16, false, false);
-    v += __uint_as_float(((lane >> 4) & 1) ? r16[0] : r16[1]);
-    v += dpp_f<0x128>(v);                     // row_ror:8
-    const float up = dpp_f<0x104>(v), dn = dpp_f<0x114>(v);   // row_shl:4, row_shr:4
-    v += (lane & 4) ? dn : up;
-    v += dpp_f<kQuadXor2>(v);
-    v += dpp_f<kQuadXor1>(v);
-    return v;
+    if constexpr (O == 32) {
+        const uint32_t b = __float_as_uint(v);
+        const auto r = __builtin_amdgcn_permlane32_swap(b, b, false, false);
+        return __uint_as_float(lane >= 32 ? r[0] : r[1]);
+    } else if constexpr (O == 16) {
+        const uint32_t b = __float_as_uint(v);
+        const auto r = __builtin_amdgcn_permlane16_swap(b, b, false, false);
+        return __uint_as_float(((lane >> 4) & 1) ? r[0] : r[1]);
+    } else if constexpr (O == 8) {
+        return dpp_f<0x128>(v);
+    } else if constexpr (O == 4) {
+        const float up = dpp_f<0x104>(v), dn = dpp_f<0x114>(v);
+        return (lane & 4) ? dn : up;
+    } else {
+        return dpp_f<O == 2 ? kQuadXor2 : kQuadXor1>(v);
+    }
 }
+
+// The xor butterfly v += v[lane ^ o] for o = FROM, .., TO, halving or
+// doubling from one to the next.
+template <int FROM, int TO>
+__device__ __forceinline__ float xor_sum(float v) {
+    v += lane_xor<FROM>(v);
+    if constexpr (FROM == TO)
+        return v;
+    else
+        return xor_sum<(FROM > TO ? FROM / 2 : FROM * 2), TO>(v);
+}
+template <int FROM, int TO>
+__device__ __forceinline__ float xor_max(float v) {
+    v = fmaxf(v, lane_xor<FROM>(v));
+    if constexpr (FROM == TO)
+        return v;
+    else
+        return xor_max<(FROM > TO ? FROM / 2 : FROM * 2), TO>(v);
+}
+
+// o = 32, 16, .., 1: every lane ends with the same sum
+__device__ __forceinline__ float xor_sum64(float v) { return xor_sum<32, 1>(v); }
 
 // Combines the four virtual-wave sums (red: LDS float[4], written by lane 0
 // of each virtual wave before the barrier inside).
