@@ -14,8 +14,9 @@
 //  * rf_gemm_q4k_f16a_kernel (Q4_K where 256 x 128 tiles fill more than half
 //    of the CUs): 4 waves, each weight dequantised once per 256 rows of A,
 //    A and the weight ring by LDS DMA.
-//  * rf_gemm_q4k_f16s_kernel (Q4_K otherwise) and rf_gemm_q6k_f16a_kernel
-//    (Q6_K from K = 768): 8 waves over 64- or 128-row x 64-column tiles, K
+//  * rf_gemm_q4k_f16s_kernel / rf_gemm_q4k_f16w_kernel (Q4_K otherwise) and
+//    rf_gemm_q6k_f16a_kernel (Q6_K from K = 768): 8 waves (16 on Q4_K's 64-row
+//    tiles) over 64- to 256-row x 64-column tiles, K
 //    sliced over waves and added through LDS; when the tiles leave at least
 //    half the CUs idle, K is also split over workgroups whose partial tiles
 //    rf_gemm_split_reduce_kernel adds in split order.
@@ -2273,6 +2274,7 @@ constexpr int kQ4sThreads = 512;
 constexpr int kQ4sBN = 64;
 constexpr int kQ4sStage = 16 * 1024;                  // 64 rows x 144 B (+ padding DMAs)
 
+// FMR = 4 (128 rows) or 8.
 // FMR = 8 (256 x 64 tiles): each weight dequantised once per 256 rows of A;
 // LDS then holds two ring stages and four 32 KB A buffers (one chunk of DMA
 // slack), as in the tall Q6_K tiles, and the K-slice partials go through
@@ -2520,6 +2522,217 @@ __device__ __forceinline__ void q4s_wg(const uint16_t* __restrict__ A, const uin
                     }
                 }
             }
+        }
+    }
+}
+
+// ── q4w: Q4_K GEMM on fp16 activations, 64 x 64 tiles on sixteen waves ────
+// (rf_gemm_q4_k_f16_launch and the launchers on it at M <= 64, and where
+// 64-row tiles come to at most one round of CUs).  A 64-row tile feeds each
+// weight to two MFMAs only, so the wave's own instruction stream (about 70
+// per 64-wide chunk: dequantisation, scales, addresses, DMA issue) and its
+// waits set the time, not a unit: with the eight waves of
+// rf_gemm_q4k_f16s_kernel, two a SIMD, ~330 ns a chunk against ~150 ns of
+// issue.  Here a step is 128 k (half a super-block) and four waves share a
+// SIMD: wave w = 8 cg + 4 kk + ks takes k [64 kk + 16 ks, +16) of the step for
+// the tile's 64 rows and the 32 columns of group cg.  A wave then needs the
+// scale and minimum of one sub-block per step, and the eight K-slice partials
+// of an output are added through LDS in slice order, each output written
+// once.  A: the step's two 64-wide chunks (XOR-swizzled 128-byte rows), six
+// buffers; weights: three super-block stages, as there.
+// Measured (us, eight waves / sixteen, fp16 A, one box): 64 x 14336 x 4096
+// 23.6 / 21.3, 64 x 4096 x 12288 22.6 / 20.8, 64 x 8448 x 3072 accumulating
+// 18.4 / 15.7, 256 x 4096 x 11264 49.1 / 45.9.  Bound now: per super-block and
+// SIMD ~1300 cycles of VALU (65 instructions a wave, the 16 v_fma_mix at half
+// rate) beside 512 of MFMA.
+constexpr int kQ4wThreads = 1024;
+constexpr int kQ4wBM = 64;
+constexpr int kQ4wRS = 3;
+constexpr int kQ4wABufs = 6;                          // DMA of step t + 5 issued in step t
+constexpr int kQ4wABuf = kQ4wBM * 2 * kKC * 2;        // 16 KB: chunk kk of the step at 8 KB kk
+constexpr int kQ4wLds = kQ4wRS * kQ4sStage + kQ4wABufs * kQ4wABuf;   // 147,456 B
+static_assert(16 * 2 * 4096 <= kQ4wLds, "the exchanged partials fit");
+
+template <bool ACC>
+__global__ __launch_bounds__(kQ4wThreads) void rf_gemm_q4k_f16w_kernel(const uint16_t* __restrict__ A,
+                                                                        const uint8_t* __restrict__ W,
+                                                                        float* __restrict__ D, int M, int N, int K,
+                                                                        const float* __restrict__ gate, KSplit sp) {
+    __shared__ __align__(16) uint8_t lds[kQ4wLds];
+    uint8_t* ring = lds;
+    uint8_t* abuf0 = lds + kQ4wRS * kQ4sStage;
+    const uint32_t ring_lds0 = (uint32_t)(size_t)(__attribute__((address_space(3))) uint8_t*)(ring);
+    const uint32_t a_lds0 = (uint32_t)(size_t)(__attribute__((address_space(3))) uint8_t*)(abuf0);
+
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int ks = wave & 3, kk = (wave >> 2) & 1, cg = wave >> 3;
+    const int h = lane >> 5, col = lane & 31;
+    const int mtiles = (M + kQ4wBM - 1) / kQ4wBM;
+    int v = xcd_remap((int)blockIdx.x, (int)gridDim.x);
+    const int nsb_row = K / kQK;
+    int sb0 = 0, nsb = nsb_row;                // this workgroup's super-blocks [sb0, sb0 + nsb) of each row
+    if (sp.S > 1) {
+        const int per = mtiles * (N / kQ4sBN);
+        const int s = v / per;
+        v -= s * per;
+        sb0 = s * nsb_row / sp.S;
+        nsb = (s + 1) * nsb_row / sp.S - sb0;
+        D = sp.part + (size_t)s * M * N;
+        gate = nullptr;
+    }
+    const int m0 = (v % mtiles) * kQ4wBM;      // the M tiles of one column tile are neighbours
+    const int n0 = (v / mtiles) * kQ4sBN;
+    const int nsteps = 2 * nsb;
+    const uint32_t row_bytes = (uint32_t)nsb_row * kQ4KBytes;
+
+    // ---- weight ring: wave w moves 16-byte pieces [64 w, 64 w + 64) of a stage
+    // (row i / 9, piece i % 9; past the stage's 576 the last one again) --------
+    const uint8_t* w_tile = W + (size_t)n0 * row_bytes + (size_t)sb0 * kQ4KBytes;
+    const uint32_t roff = tid < 576 ? (uint32_t)(tid / 9) * row_bytes + 16u * (uint32_t)(tid % 9)
+                                    : 63u * row_bytes + 128u;
+    auto w_dma = [&](int sb) {
+        lds_dma16(ring_lds0 + (uint32_t)(sb % kQ4wRS) * kQ4sStage + 1024u * (uint32_t)wave, roff,
+                  w_tile + (size_t)min(sb, nsb - 1) * kQ4KBytes);
+    };
+
+    // ---- A: wave w moves rows 8 (w % 8) + L / 8 of chunk w / 8 of a step,
+    // position L % 8 (k piece (L % 8) ^ g(row)); M % 64 == 0 --------------------
+    const uint8_t* a_tile = reinterpret_cast<const uint8_t*>(A) + ((size_t)m0 * K + (size_t)sb0 * kQK) * 2;
+    const int ar = 8 * (wave & 7) + (lane >> 3);
+    const uint32_t a_voff =
+        (uint32_t)(ar * K + kKC * (wave >> 3) + 8 * ((lane & 7) ^ (ar & 7) ^ ((ar >> 3) & 1))) * 2u;
+    auto a_dma = [&](int t, int buf) {
+        lds_dma16(a_lds0 + (uint32_t)(buf * kQ4wABuf + wave * 1024), a_voff,
+                  a_tile + (size_t)min(t, nsteps - 1) * 2 * kKC * 2);
+    };
+
+    // ---- B: the lane's weight row (column 32 cg + col) in the ring stage ------
+    const int brow = 32 * cg + col;
+    const int hf = ks >> 1;                     // high nibbles (odd sub-block) for ks >= 2
+    const uint32_t nmask = hf ? 0x00F000F0u : 0x000F000Fu;
+    const float nfac = hf ? 1048576.0f : 16777216.0f;
+    const int sbyte = 8 * (2 * kk + hf);        // step HQ takes sub-block 4 HQ + 2 kk + hf
+    float sD[2], sM[2];                         // per step of the super-block: (d sc 2^x, -dmin m)
+    auto hdr_read = [&](int sb) {
+        const u32x4 hd = *reinterpret_cast<const u32x4*>(ring + (sb % kQ4wRS) * kQ4sStage + brow * kQ4KBytes);
+        const float d = half_bits_to_float(hd.x) * nfac, dmin = half_bits_to_float(hd.x >> 16);
+        // get_scale_min_k4, one byte of the low and one of the high sub-blocks
+        const uint32_t y = hd.y >> sbyte, z = hd.z >> sbyte, w = hd.w >> sbyte;
+        const uint32_t sc[2] = {y & 0x3Fu, (w & 0x0Fu) | ((y >> 2) & 0x30u)};
+        const uint32_t mn[2] = {z & 0x3Fu, ((w >> 4) & 0x0Fu) | ((z >> 2) & 0x30u)};
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            sD[q] = d * (float)sc[q];
+            sM[q] = -(dmin * (float)mn[q]);
+        }
+    };
+    u32x2 rqs;
+    auto qs_read = [&](int q, int sb) {
+        rqs = *reinterpret_cast<const u32x2*>(ring + (sb % kQ4wRS) * kQ4sStage + brow * kQ4KBytes + 16 + 64 * q +
+                                              32 * kk + 16 * (ks & 1) + 8 * h);
+    };
+    u32x4 bq[2];                          // [step parity]
+    auto b_dequant = [&](int q) {
+        const uint2 a = f16a_dq4(rqs.x, nmask, sD[q], sM[q]);
+        const uint2 b = f16a_dq4(rqs.y, nmask, sD[q], sM[q]);
+        bq[q] = u32x4{a.x, a.y, b.x, b.y};
+    };
+
+    f32x16 acc[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) acc[i][e] = 0.0f;
+
+    const uint32_t foff = (uint32_t)(kk * (kQ4wABuf / 2) + col * 128 +
+                                     16 * ((2 * ks + h) ^ (col & 7) ^ ((col >> 3) & 1)));
+    f16x8 af[2][2];
+    auto frag_ld = [&](int set, int buf, int i) {
+        af[set][i] = *reinterpret_cast<const f16x8*>(abuf0 + buf * kQ4wABuf + foff + 32 * i * 128);
+    };
+
+    // ---- prologue: ring stages 0, 1; A steps 0 .. 4; step 0's operands --------
+    w_dma(0);
+    w_dma(1);
+#pragma unroll
+    for (int t = 0; t < kQ4wABufs - 1; ++t) a_dma(t, t);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    lds_barrier();
+    hdr_read(0);
+    qs_read(0, 0);
+    b_dequant(0);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) frag_ld(0, 0, i);
+
+    // Step t = 2 sb + HQ: A buffer t % 6, ring stage sb % 3.  After the first
+    // MFMA every LDS read of step t + 1; the A DMA of step t + 5 into the buffer
+    // step t - 1 used (its fragments were read in step t - 2); in HQ 0 the ring
+    // DMA of super-block sb + 2 into the stage sb - 1 used (last read in step
+    // 2 sb - 2).  What step t + 1 reads for step t + 2 must have landed at the end
+    // of step t: A of step t + 2, issued in t - 3 (in flight behind it: the A of
+    // t - 2, t - 1, t and one ring DMA, 4; after an HQ 0 step at most 3, because:)
+    // and, for HQ 0, super-block sb + 1's stage, issued in t - 2, with A(t - 1),
+    // A(t) and ring(t) behind it.
+    int ab = 0;
+    auto iteration = [&](auto hqc, int sb) {
+        constexpr int HQ = decltype(hqc)::value;
+        const int t = 2 * sb + HQ;
+        const int sbn = HQ ? sb + 1 : sb;
+        const int abn = ab == kQ4wABufs - 1 ? 0 : ab + 1;
+        const int abp = ab == 0 ? kQ4wABufs - 1 : ab - 1;
+        acc[0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[HQ][0], __builtin_bit_cast(f16x8, bq[HQ]), acc[0], 0, 0, 0);
+        if constexpr (HQ == 1) hdr_read(sbn);
+        qs_read(HQ ^ 1, sbn);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) frag_ld(HQ ^ 1, abn, i);
+        a_dma(t + kQ4wABufs - 1, abp);
+        __builtin_amdgcn_sched_barrier(0);
+        acc[1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[HQ][1], __builtin_bit_cast(f16x8, bq[HQ]), acc[1], 0, 0, 0);
+        if constexpr (HQ == 0) w_dma(sb + 2);
+        b_dequant(HQ ^ 1);
+        __builtin_amdgcn_sched_barrier(0);
+        asm volatile("s_waitcnt vmcnt(%0)" :: "n"(HQ ? 4 : 3) : "memory");
+        lds_barrier();
+        ab = abn;
+    };
+    for (int sb = 0; sb < nsb; ++sb) {
+        iteration(std::integral_constant<int, 0>{}, sb);
+        iteration(std::integral_constant<int, 1>{}, sb);
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+
+    // ---- K slices: every wave parks its two blocks in LDS ([wave][block][e / 4]
+    // [lane] of float4); wave (cg, b, q) adds rows 8 q .. + 7 of block b of column
+    // group cg over the slices 0 .. 7 in that order ------------------------------
+    float4* xch = reinterpret_cast<float4*>(lds);
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            xch[((wave * 2 + i) * 4 + q) * 64 + lane] =
+                make_float4(acc[i][4 * q], acc[i][4 * q + 1], acc[i][4 * q + 2], acc[i][4 * q + 3]);
+    __syncthreads();
+    const int b = (wave >> 2) & 1, q = wave & 3;
+    float s4[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int src = 0; src < 8; ++src) {
+        const float4 p = xch[(((8 * cg + src) * 2 + b) * 4 + q) * 64 + lane];
+        s4[0] += p.x;
+        s4[1] += p.y;
+        s4[2] += p.z;
+        s4[3] += p.w;
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        const size_t e = (size_t)(m0 + 32 * b + 8 * q + 4 * h + u) * N + n0 + brow;
+        if (!ACC && gate != nullptr) {           // up projection of a SwiGLU: fp16 silu(gate) * up
+            const float gg = gate[e];
+            reinterpret_cast<uint16_t*>(D)[e] = f16_bits_rn(gg / (1.0f + expf(-gg)) * s4[u]);
+        } else {
+            D[e] = ACC ? D[e] + s4[u] : s4[u];
         }
     }
 }
@@ -2903,10 +3116,11 @@ static void reduce_for(bool acc, const float* G, const float* part, int S, int M
 }
 
 // Q4_K on fp16 activations: 256 x 128 tiles (rf_gemm_q4k_f16a_kernel) where
-// they fill more than half the CUs, else the eight-wave
-// K-sliced tiles (rf_gemm_q4k_f16s_kernel) of 256 rows (from M =
-// kQ4TallMinM: each weight dequantised once per 256 rows), 64 rows (M <= 64,
-// or when they come to at most one round of CUs) or 128, split over K when
+// they fill more than half the CUs, else the K-sliced tiles: eight waves
+// (rf_gemm_q4k_f16s_kernel) on 256 rows (from M =
+// kQ4TallMinM: each weight dequantised once per 256 rows) or 128, sixteen
+// (rf_gemm_q4k_f16w_kernel) on 64 (M <= 64,
+// or when they come to at most one round of CUs), split over K when
 // they leave at least half the CUs idle and `part` is given.
 // G: when given, D receives fp16 silu(G) * (A W^T) (the up projection of a
 // SwiGLU whose gate product G [M x N] is already computed)
@@ -2921,13 +3135,20 @@ static void q4_f16_tiles(const uint16_t* A, const uint8_t* w, float* D, int M, i
                          const float* G, const PartBuf& part, const RowNorm* rn = nullptr) {
     const long tiles = (long)((M + 32 * FMR - 1) / (32 * FMR)) * (N / kQ4sBN);
     const int S = 2 * tiles <= (long)device_cu_count() ? ksplit_count(tiles, K / kQK, M, N, part) : 1;
+    auto go = [&](auto accc, float* d, const float* g, const KSplit& sp) {
+        constexpr bool kAcc = decltype(accc)::value;
+        const dim3 grid((unsigned)(tiles * sp.S));
+        if constexpr (FMR == 2)
+            hipLaunchKernelGGL(rf_gemm_q4k_f16w_kernel<kAcc>, grid, dim3(kQ4wThreads), 0, st, A, w, d, M, N, K, g, sp);
+        else
+            hipLaunchKernelGGL((rf_gemm_q4k_f16s_kernel<FMR, kAcc>), grid, dim3(kQ4sThreads), 0, st, A, w, d, M, N, K,
+                               g, sp);
+    };
     if (S > 1) {
-        hipLaunchKernelGGL((rf_gemm_q4k_f16s_kernel<FMR, false>), dim3((unsigned)(tiles * S)), dim3(kQ4sThreads), 0,
-                           st, A, w, nullptr, M, N, K, nullptr, KSplit{S, part.p});
+        go(std::false_type{}, nullptr, nullptr, KSplit{S, part.p});
         reduce_for(ACC, G, part.p, S, M, N, D, st, rn);
     } else {
-        hipLaunchKernelGGL((rf_gemm_q4k_f16s_kernel<FMR, ACC>), dim3((unsigned)tiles), dim3(kQ4sThreads), 0, st, A, w,
-                           D, M, N, K, G, KSplit{1, nullptr});
+        go(std::bool_constant<ACC>{}, D, G, KSplit{1, nullptr});
     }
 }
 
