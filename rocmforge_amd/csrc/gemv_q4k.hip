@@ -22,7 +22,8 @@
 //  * Long rows (K a multiple of 4096 from 8192: the Qwen3-8B ffn_down) take
 //    a K-split kernel instead (rf_q4k_q8_lin_kernel): each wave of a team
 //    keeps its K slice's Q8 x in registers and streams every row of its
-//    workgroup.
+//    workgroup.  Other K above 8192 take it (rf_q4k_q8_any_kernel, same
+//    bits as the row steps) where the rows fill the steps badly.
 #include <type_traits>
 
 #include "q6k_lin.h"
@@ -102,6 +103,19 @@ __device__ __forceinline__ float q4k_q8_unit_dot(const Q4KUnit& u, int p, const 
     acc = q4k_q8_combine(acc, xd0, d, dmin, sc0, m0, dlo, qs0);
     acc = q4k_q8_combine(acc, xd1, d, dmin, sc1, m1, dhi, qs1);
     return acc;
+}
+
+// The two terms alone, before the activations' scales.
+__device__ __forceinline__ float2 q4k_q8_unit_terms(const Q4KUnit& u, int p, const u32x4 xlo[2], const u32x4 xhi[2],
+                                                    int qs0, int qs1) {
+    int dlo, dhi;
+    q4k_int_dots(u, xlo, xhi, &dlo, &dhi);
+    const float d = half_bits_to_float(u.hdr.x);
+    const float dmin = half_bits_to_float(u.hdr.x >> 16);
+    int sc0, m0, sc1, m1;
+    q4k_scale_min_pair(u.hdr.y, u.hdr.z, u.hdr.w, p, &sc0, &m0, &sc1, &m1);
+    return make_float2(d * (float)sc0 * (float)dlo - dmin * (float)m0 * (float)qs0,
+                       d * (float)sc1 * (float)dhi - dmin * (float)m1 * (float)qs1);
 }
 
 // ONE: K <= 4096 (a row group is one pipeline step), so the step -> (row
@@ -383,6 +397,40 @@ __global__ __launch_bounds__(kThreads) void rf_q4k_f32_gemv_kernel(const uint8_t
     }
 }
 
+// The 64 floats v as two Q8_0 blocks in a lane's registers: the quantiser's
+// arithmetic (q8_quantize_batch) with no cross-lane step.
+__device__ __forceinline__ void q8_quantize_lane(const float4 (&v)[16], u32x4 (&xlo)[2], u32x4 (&xhi)[2],
+                                                 float (&xd)[2], int (&xq)[2]) {
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+        float e[32];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            e[4 * i] = v[8 * b + i].x; e[4 * i + 1] = v[8 * b + i].y;
+            e[4 * i + 2] = v[8 * b + i].z; e[4 * i + 3] = v[8 * b + i].w;
+        }
+        float amax = 0.0f;
+#pragma unroll
+        for (int i = 0; i < 32; ++i) amax = fmaxf(amax, fabsf(e[i]));
+        const float scale = fmaxf(amax / 127.0f, 1e-30f);
+        const float sf = __half2float(__float2half(scale));
+        const float inv = 1.0f / sf;
+        uint32_t packed[8] = {0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u};
+        int sum = 0;
+#pragma unroll
+        for (int i = 0; i < 32; ++i) {
+            const int q = (int)fminf(fmaxf(e[i] * inv, -127.0f), 127.0f);
+            sum += q;
+            packed[i >> 2] |= ((uint32_t)q & 0xFFu) << (8 * (i & 3));
+        }
+        u32x4* dst = b ? xhi : xlo;
+        dst[0] = u32x4{packed[0], packed[1], packed[2], packed[3]};
+        dst[1] = u32x4{packed[4], packed[5], packed[6], packed[7]};
+        xd[b] = sf;
+        xq[b] = sum;
+    }
+}
+
 // ── K-split Q4_K Q8-inline GEMV for long rows (K >= 8192, K / 256 % 16 == 0) ──
 // A team of nwk = K / 4096 waves per workgroup; team wave tw takes
 // super-blocks [16 tw, 16 tw + 16) of every row (lane 4 s + p: super-block
@@ -417,47 +465,17 @@ __global__ __launch_bounds__(512) void rf_q4k_q8_lin_kernel(const uint8_t* __res
     u32x4 xlo[2], xhi[2];
     float xd[2];
     int xq[2];
-    {
-        const float4* xv = reinterpret_cast<const float4*>(x + (size_t)sb * kQK + 64 * p);
-        float4 v[16];
+    const float4* xv = reinterpret_cast<const float4*>(x + (size_t)sb * kQK + 64 * p);
+    float4 v[16];
 #pragma unroll
-        for (int i = 0; i < 16; ++i) v[i] = xv[i];
-        if (norm_w) {
-            const float4* gv = reinterpret_cast<const float4*>(norm_w + (size_t)sb * kQK + 64 * p);
+    for (int i = 0; i < 16; ++i) v[i] = xv[i];
+    if (norm_w) {
+        const float4* gv = reinterpret_cast<const float4*>(norm_w + (size_t)sb * kQK + 64 * p);
 #pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                const float4 gg = gv[i];
-                v[i] = make_float4((v[i].x * inv_rms) * gg.x, (v[i].y * inv_rms) * gg.y, (v[i].z * inv_rms) * gg.z,
-                                   (v[i].w * inv_rms) * gg.w);
-            }
-        }
-#pragma unroll
-        for (int b = 0; b < 2; ++b) {
-            float e[32];
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                e[4 * i] = v[8 * b + i].x; e[4 * i + 1] = v[8 * b + i].y;
-                e[4 * i + 2] = v[8 * b + i].z; e[4 * i + 3] = v[8 * b + i].w;
-            }
-            float amax = 0.0f;
-#pragma unroll
-            for (int i = 0; i < 32; ++i) amax = fmaxf(amax, fabsf(e[i]));
-            const float scale = fmaxf(amax / 127.0f, 1e-30f);
-            const float sf = __half2float(__float2half(scale));
-            const float inv = 1.0f / sf;
-            uint32_t packed[8] = {0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u};
-            int sum = 0;
-#pragma unroll
-            for (int i = 0; i < 32; ++i) {
-                const int q = (int)fminf(fmaxf(e[i] * inv, -127.0f), 127.0f);
-                sum += q;
-                packed[i >> 2] |= ((uint32_t)q & 0xFFu) << (8 * (i & 3));
-            }
-            u32x4* dst = b ? xhi : xlo;
-            dst[0] = u32x4{packed[0], packed[1], packed[2], packed[3]};
-            dst[1] = u32x4{packed[4], packed[5], packed[6], packed[7]};
-            xd[b] = sf;
-            xq[b] = sum;
+        for (int i = 0; i < 16; ++i) {
+            const float4 gg = gv[i];
+            v[i] = make_float4((v[i].x * inv_rms) * gg.x, (v[i].y * inv_rms) * gg.y, (v[i].z * inv_rms) * gg.z,
+                               (v[i].w * inv_rms) * gg.w);
         }
     }
     const uint8_t* wl = w + (size_t)sb * kQ4KBytes;
@@ -471,12 +489,93 @@ __global__ __launch_bounds__(512) void rf_q4k_q8_lin_kernel(const uint8_t* __res
         if ((lane & 15) == 0) part[(j * nwk + tw) * 4 + (lane >> 4)] = r16;
     };
     Q4KUnit ring[NB];
-    ring_pipeline<NB>(nrows, ring, load, process, [&]() {});
+    ring_pipeline<NB>(nrows, ring, load, process, [&]() { q8_quantize_lane(v, xlo, xhi, xd, xq); });
     __syncthreads();
     for (int j = tw * kWave + lane; j < nrows; j += nwk * kWave) {
         float t = 0.0f;
         for (int k = 0; k < 4 * nwk; ++k) t += part[j * nwk * 4 + k];
         y[g + j * G] = t + (residual ? residual[g + j * G] : 0.0f);
+    }
+}
+
+// The same split for any K, with the sums of the one-row-per-step kernel bit
+// for bit: there a lane adds its terms xd (d sc dot - dmin m sum) of all slices
+// in one chain, so a wave leaves its lanes' two terms (before xd) in LDS and
+// the chains run after the loop.  The last slice may be short; lanes past the
+// row's end load its last super-block and are left out.  x is quantised behind
+// the first rows' loads (ahead of them 0.1-0.6 us slower).  Bound: the weight
+// stream with three rows in flight a wave; what it saves over the other kernel
+// is that every wave of the grid has rows to the end (a row a step, N / CUs of
+// them) and no Q8 pass through LDS.  us, one-row-per-step kernel / this one,
+// + residual, weights beyond the Infinity Cache: 2304 x 9216 8.6 / 6.7,
+// 2560 x 9728 8.7 / 6.9, 1536 x 8960 6.3 / 5.9, 3584 x 18944 12.4 / 12.0,
+// 5120 x 13824 12.8 / 12.0, 5120 x 25600 20.9 / 19.3, 17 x 18944 7.7 / 6.1.
+template <int NB>
+__global__ __launch_bounds__(512) void rf_q4k_q8_any_kernel(const uint8_t* __restrict__ w,
+                                                             const float* __restrict__ x, const float* residual,
+                                                             float* y, int K, int N) {
+    extern __shared__ __align__(16) float2 terms[];   // [nwk][64] xd, then [rows of this workgroup][nwk][64]
+    const int lane = threadIdx.x & (kWave - 1);
+    const int tw = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const int nwk = blockDim.x / kWave;
+    const int nsb = K / kQK;
+    const size_t row_bytes = (size_t)nsb * kQ4KBytes;
+    const int s = lane >> 2, p = lane & 3;
+    const int sb = min(16 * tw + s, nsb - 1);
+    const int g = blockIdx.x, G = gridDim.x;
+    const int nrows = g < N ? (N - 1 - g) / G + 1 : 0;
+    float2* tl = terms + nwk * kWave + tw * kWave + lane;   // row j at + j nwk 64
+
+    u32x4 xlo[2], xhi[2];
+    float xd[2];
+    int xq[2];
+    const float4* xv = reinterpret_cast<const float4*>(x + (size_t)sb * kQK + 64 * p);
+    float4 v[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) v[i] = xv[i];
+    const uint8_t* wl = w + (size_t)sb * kQ4KBytes;
+    auto load = [&](Q4KUnit& u, int j) {
+        const int row = nrows ? g + min(j, nrows - 1) * G : 0;
+        u = q4k_load_unit(wl + (size_t)row * row_bytes, p);
+    };
+    auto process = [&](const Q4KUnit& u, int j) {
+        tl[j * nwk * kWave] = q4k_q8_unit_terms(u, p, xlo, xhi, xq[0], xq[1]);
+    };
+    Q4KUnit ring[NB];
+    ring_pipeline<NB>(nrows, ring, load, process, [&]() {
+        q8_quantize_lane(v, xlo, xhi, xd, xq);
+        terms[tw * kWave + lane] = make_float2(xd[0], xd[1]);
+    });
+    __syncthreads();
+    // wave tw takes rows tw, tw + nwk, .., four chains at a time; lane u ends
+    // with the u-th row's sum of a run of 64
+    for (int j0 = tw; j0 < nrows; j0 += 64 * nwk) {
+        const int jl = j0 + lane * nwk;
+        const float r = residual && jl < nrows ? residual[g + jl * G] : 0.0f;
+        float mine = 0.0f;
+        for (int u0 = 0; u0 < 64 && j0 + u0 * nwk < nrows; u0 += 4) {
+            float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+            for (int k = 0; k < nwk; ++k) {
+                const float2 d = terms[k * kWave + lane];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int j = min(j0 + (u0 + i) * nwk, nrows - 1);
+                    const float2 t = terms[((1 + j) * nwk + k) * kWave + lane];
+                    const float a = __builtin_fmaf(d.y, t.y, __builtin_fmaf(d.x, t.x, acc[i]));
+                    acc[i] = 16 * k + s < nsb ? a : acc[i];
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const float r16 = row16_sum(acc[i]);
+                auto row = [&](int l) {
+                    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, r16), l));
+                };
+                const float sum = (row(0) + row(16)) + (row(32) + row(48));   // on all lanes, before the select
+                mine = lane == u0 + i ? sum : mine;
+            }
+        }
+        if (jl < nrows) y[g + jl * G] = residual ? mine + r : mine;
     }
 }
 
@@ -632,6 +731,27 @@ static hipError_t launch_q4_lin(const void* w, const float* x, const float* res,
     return hipGetLastError();
 }
 
+// Other K above 8192 where the one-row-per-step kernel's last step, two rows for
+// each of its 4 CUs waves, leaves at least an eighth of all its row slots empty
+// (rf_q4k_q8_any_kernel, the same bits; figures there).  With the slots full it
+// is the slower one from three slices of K up (us, row steps / this: 4096 x
+// 11008 9.0 / 9.4, 8192 x 18944 20.6 / 22.0), and with two slices it has too few
+// waves (2560 x 6912 6.0 / 6.8, 4096 x 5120 6.2 / 8.2).  false: not launched.
+static bool launch_q4_any(const void* w, const float* x, const float* res, float* y, int K, int N, hipStream_t st,
+                          hipError_t* e) {
+    const int cap = device_cu_count();
+    const long step = 8L * cap, slots = (N + step - 1) / step * step;
+    if (K <= 8192 || !aligned16(x) || 8L * N > 7 * slots) return false;
+    const int nwk = (K + 4095) / 4096;
+    const int grid = N < cap ? N : cap;
+    const size_t lds = ((size_t)((N + grid - 1) / grid) + 1) * nwk * kWave * sizeof(float2);
+    if (lds > 160 * 1024) return false;
+    hipLaunchKernelGGL((rf_q4k_q8_any_kernel<kQ4LinRing>), dim3(grid), dim3(nwk * 64), lds, st,
+                       static_cast<const uint8_t*>(w), x, res, y, K, N);
+    *e = hipGetLastError();
+    return true;
+}
+
 extern "C" hipError_t gemv_q4_k_f32_q8_inline_launch(const void* weights_q4_k, const float* input, float* output,
                                                      int n_rows, int ncols_dst, hipStream_t stream) {
     if (n_rows <= 0 || ncols_dst <= 0) return hipErrorInvalidValue;
@@ -640,6 +760,8 @@ extern "C" hipError_t gemv_q4_k_f32_q8_inline_launch(const void* weights_q4_k, c
     if (!aligned16(weights_q4_k)) return hipErrorInvalidValue;
     if (q4_lin_ok(weights_q4_k, input, n_rows))
         return launch_q4_lin(weights_q4_k, input, nullptr, output, n_rows, ncols_dst, stream);
+    hipError_t e;
+    if (launch_q4_any(weights_q4_k, input, nullptr, output, n_rows, ncols_dst, stream, &e)) return e;
     return launch_q8<kPlain>(weights_q4_k, nullptr, input, nullptr, output, n_rows, ncols_dst, stream);
 }
 
@@ -652,6 +774,8 @@ extern "C" hipError_t gemv_q4_k_f32_q8_inline_residual_launch(const void* weight
     if (!aligned16(weights_q4_k)) return hipErrorInvalidValue;
     if (q4_lin_ok(weights_q4_k, input, n_rows))
         return launch_q4_lin(weights_q4_k, input, residual, output, n_rows, ncols_dst, stream);
+    hipError_t e;
+    if (launch_q4_any(weights_q4_k, input, residual, output, n_rows, ncols_dst, stream, &e)) return e;
     return launch_q8<kResidual>(weights_q4_k, nullptr, input, residual, output, n_rows, ncols_dst, stream);
 }
 
