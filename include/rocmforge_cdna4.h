@@ -106,8 +106,9 @@ hipError_t gemv_q6_k_f32_residual_launch(const void* weights_q6_k, const float* 
  * capture, the slot of an idle stream (hipStreamQuery), else the
  * fp32-activation tiles run (same values up to summation order).  A stream
  * that will be captured should launch a GEMM once before its capture, so
- * that it holds a slot.  Q6_K takes the fp16 tiles when
- * K % 2048 == 0 and the weights are 16-byte aligned. */
+ * that it holds a slot.  Q6_K takes the fp16 tiles when the weights are
+ * 16-byte aligned and K % 2048 == 0, or K >= 768 with a 16-byte aligned
+ * output. */
 hipError_t wmma_gemm_q4_k_launch(const float* input, const void* weights_q4_k, float* output, int M, int N, int K,
                                  hipStream_t stream);
 hipError_t wmma_gemm_q6_k_launch(const float* input, const void* weights_q6_k, float* output, int M, int N, int K,

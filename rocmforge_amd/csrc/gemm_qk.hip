@@ -3222,7 +3222,8 @@ static hipError_t gemm_q4_f16(const uint16_t* A, const void* W, float* D, int M,
 // Q6_K on fp16 activations (rf_gemm_q6k_f16a_kernel): 256 x 64 tiles from
 // M = kQ6TallMinM rows (each weight dequantised once per 256 rows), else
 // 128 x 64, split over K as gemm_q4_f16 does.  The caller has checked
-// M % 64, N % 64, K % 2048 and 16-byte alignment of A and W.
+// M % 64, N % 64 and 16-byte alignment of A and W (and of D with ANY, whose
+// K is any multiple of 256; otherwise K % 2048 == 0).
 #ifndef RF_Q6_TALL_MIN_M
 #define RF_Q6_TALL_MIN_M 256
 #endif
