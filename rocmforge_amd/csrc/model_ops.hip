@@ -1937,8 +1937,10 @@ void rf_attn_prefill_kernel(const _Float16* __restrict__ Q, const _Float16* __re
     typedef uint32_t u4 __attribute__((ext_vector_type(4)));
     const uint32_t sign = scale < 0.0f ? 0x80008000u : 0u;
     h8 qf[8];
-    // (1e-30: a scale of zero keeps every weight at one and the masked ones at zero)
-    const float scale2 = fmaxf(fabsf(scale) * 1.4426950408889634f, 1e-30f);   // log2 e
+    // (1e-30: a scale of zero keeps every weight at one and the masked ones at zero;
+    // a NaN stays one)
+    const float scale_l2 = fabsf(scale) * 1.4426950408889634f;   // log2 e
+    const float scale2 = scale_l2 < 1e-30f ? 1e-30f : scale_l2;
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
         const u4 w = *reinterpret_cast<const u4*>(Q + (size_t)(q0 + col) * qrow + (size_t)head * kAttD + 16 * k + 8 * hi);

@@ -90,3 +90,9 @@ def test_maximum_rising_tile_by_tile(rf, dev):
     got = run(rf, q, k, v, 1, scale)
     ref, mag = reference(q, k, v, 1, scale)
     assert bool(((got - ref).abs() <= 1.25 * U16 * mag + 1e-5).all())
+
+
+@pytest.mark.parametrize("seq,nq,nkv", [(64, 2, 1), (2048, 64, 8), (4096, 32, 8)])
+def test_a_nan_scale_gives_nan(rf, dev, seq, nq, nkv):
+    q, k, v = inputs(seq, nq, nkv, seed=11)
+    assert bool(run(rf, q, k, v, 1, math.nan).isnan().all())
