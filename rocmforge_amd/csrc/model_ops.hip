@@ -1871,6 +1871,7 @@ typedef float f16v __attribute__((ext_vector_type(16)));
 constexpr int kAttD = 128;
 constexpr uint32_t kAttRow = 2 * kAttD;          // bytes of a K / V row in LDS
 constexpr uint32_t kAttTile = 64 * kAttRow;      // one 64-key tile of K or of V
+constexpr float kAttFar = 128.0f;                // |m| from which scores are rounded before the exp
 
 // NW waves as NW / KS units times KS key groups: group g takes the tiles
 // t % KS == g and the groups' partial (m, l, O) are merged through LDS (more
@@ -1952,6 +1953,7 @@ void rf_attn_prefill_kernel(const _Float16* __restrict__ Q, const _Float16* __re
 #pragma unroll
         for (int e = 0; e < 16; ++e) o[b][e] = 0.0f;
     float m = kNegMax, l = 0.0f;
+    uint64_t far = 0;                            // lanes whose |m| is at least kAttFar
     const int query = q0 + col;
 
     // operand addresses: K lane (row col, piece 2 k + hi) in slot piece ^ (col %
@@ -2023,7 +2025,12 @@ void rf_attn_prefill_kernel(const _Float16* __restrict__ Q, const _Float16* __re
         // O is rescaled only where some lane's maximum moved.  (A maximum left behind
         // by up to 2^8 saves 6 % of the time, but then a row's largest weight is no
         // longer exactly one and peaked rows lose half their precision.)
-        if (__builtin_amdgcn_ballot_w64(tmax > m)) {
+        // exp(x - m) is 2^(s scale log2 e - m log2 e): one fma, one v_exp_f32.  m is a
+        // rounded product and the fma's is not, so the largest weight is 2^(+-2^-18) at
+        // |m| below kAttFar, but would leave fp16's range from |m| = 2^28 on: far from
+        // zero the scores are rounded as m is (in this branch, taken on every tile then).
+        float mul = scale2;
+        if (__builtin_amdgcn_ballot_w64(tmax > m) | far) {
             const float m_new = fmaxf(m, tmax);
             const float alpha = __builtin_amdgcn_exp2f(m - m_new);
             m = m_new;
@@ -2032,15 +2039,22 @@ void rf_attn_prefill_kernel(const _Float16* __restrict__ Q, const _Float16* __re
             for (int b = 0; b < 4; ++b)
 #pragma unroll
                 for (int e = 0; e < 16; ++e) o[b][e] *= alpha;
+            far = __builtin_amdgcn_ballot_w64(fabsf(m) >= kAttFar);
+            if (far) {
+#pragma unroll
+                for (int b = 0; b < 2; ++b)
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) s[b][e] = __fmul_rn(s[b][e], scale2);
+                mul = 1.0f;
+            }
         }
-        // exp(x - m) as 2^(s scale log2 e - m log2 e): one fma, one v_exp_f32
         float rs = 0.0f;
         h8 p[4];   // B operands, k-step j = (block j / 2, keys 16 (j % 2) ..)
 #pragma unroll
         for (int b = 0; b < 2; ++b)
 #pragma unroll
             for (int e = 0; e < 16; ++e) {
-                const float ex = __builtin_amdgcn_exp2f(__builtin_fmaf(s[b][e], scale2, -m));
+                const float ex = __builtin_amdgcn_exp2f(__builtin_fmaf(s[b][e], mul, -m));
                 rs += ex;
                 p[2 * b + (e >> 3)][e & 7] = (_Float16)ex;
             }

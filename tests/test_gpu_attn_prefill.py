@@ -96,3 +96,26 @@ def test_maximum_rising_tile_by_tile(rf, dev):
 def test_a_nan_scale_gives_nan(rf, dev, seq, nq, nkv):
     q, k, v = inputs(seq, nq, nkv, seed=11)
     assert bool(run(rf, q, k, v, 1, math.nan).isnan().all())
+
+
+@pytest.mark.parametrize("seq,nq,nkv", [(64, 2, 1), (512, 4, 2), (2048, 64, 8), (4096, 32, 8)])
+@pytest.mark.parametrize("size", [16.0, 300.0, 8000.0, 60000.0])
+@pytest.mark.parametrize("sign", [1.0, -1.0])
+def test_large_scores(rf, dev, seq, nq, nkv, size, sign):
+    # scores of up to +-128 size^2 scale (4e10), a multiple of each key's own size
+    q, k, v = inputs(seq, nq, nkv, seed=13)
+    q = torch.full_like(q, sign * size)
+    k = (size * (1 - 0.1 * k[:, :, :1].float().abs())).expand(k.shape).half()
+    scale = 1.0 / math.sqrt(D)
+    got = run(rf, q, k, v, 1, scale)
+    ref, mag = reference(q, k, v, 1, scale)
+    # where a row's best score leads by more than the fp32 roundings of a score (the
+    # dot of 128 terms, the scale: 2^-15 of it) and by a weight of e^-40, the row is
+    # that key's V with a weight of exactly one
+    s = (q[:, 0].double() @ k[:, 0].double().T) * scale
+    top = s.masked_fill(torch.ones(seq, seq, dtype=torch.bool, device="cuda").triu(1), -math.inf).topk(2, 1).values
+    clear = top[:, 0] - top[:, 1] > 40 + 2.0 ** -15 * top[:, 0].abs()
+    assert bool(got.isfinite().all()) and int(clear.sum()) > 0
+    group = nq // nkv
+    bound = 1e-3 * U16 * mag[:, :group] + 1e-6
+    assert bool(((got - ref)[:, :group].abs() <= bound)[clear].all())
