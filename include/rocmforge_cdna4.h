@@ -461,7 +461,9 @@ hipError_t gpu_flash_attn_decode_strided_multi_head_state(float* d_out, const fl
  * rf_flash_attn_decode_workspace_bytes(num_heads, head_dim) bytes (a smaller
  * one is rejected).  Same results as the launchers above within fp32
  * rounding; GQA groups larger than 8 take the one-workgroup path.  Launches
- * that share a workspace must be stream-ordered. */
+ * that share a workspace must be stream-ordered.  The caches of these and the
+ * folded launchers below may lie on any 2-byte address; on 16-byte addresses
+ * long sequences (head_dim 128) are read faster. */
 size_t rf_flash_attn_decode_workspace_bytes(const int num_heads, const int head_dim);
 hipError_t rf_flash_attn_decode_ws(float* d_out, const float* d_q, const uint16_t* d_k_cache, const uint16_t* d_v_cache,
                                    const int seq_len, const int num_heads, const int num_kv_heads, const int head_dim,

@@ -636,7 +636,9 @@ struct QkStep {
     const float2* cs;      // cos / sin table (rf_rope_cos_sin_kernel), or null
 };
 
-template <int LPP, bool QK>
+// RING: long sequences take the ring (its LDS is part of every launch of the
+// instance); its 16-byte DMA needs caches on 16-byte addresses.
+template <int LPP, bool QK, bool RING>
 __global__ __launch_bounds__(512) void rf_attn_split_kernel(const float* __restrict__ q,
                                                             const __half* kc,    // not restrict: QK writes a row
                                                             const __half* vc,
@@ -648,7 +650,8 @@ __global__ __launch_bounds__(512) void rf_attn_split_kernel(const float* __restr
     constexpr int NI = kSplitChunk / PPW;       // load instructions per chunk (K and V each)
     __shared__ u32x4 new_kv[2][LPP];            // QK: the new position's fp16 K and V row of this kv head
     __shared__ __align__(16) float2 lcs[QK ? 8 : 1][QK ? D / 2 : 2];   // QK: each wave's cos / sin
-    __shared__ __align__(16) uint8_t ring[LPP == 16 ? kLongStages * 2 * kLongHalf : 16];
+    __shared__ __align__(16) uint8_t ring[RING ? kLongStages * 2 * kLongHalf : 16];
+    static_assert(!RING || LPP == 16, "the ring is laid out for D = 128");
     const int seq = len_ptr ? *len_ptr : len0;
     const int kvh = blockIdx.x, split = blockIdx.y;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -779,7 +782,7 @@ __global__ __launch_bounds__(512) void rf_attn_split_kernel(const float* __restr
                 }
             }
         }
-        if constexpr (LPP == 16) {
+        if constexpr (RING) {
             typedef _Float16 h8r __attribute__((ext_vector_type(8)));
             float t[8];
 #pragma unroll
@@ -819,7 +822,7 @@ __global__ __launch_bounds__(512) void rf_attn_split_kernel(const float* __restr
         }
     };
     const int first_c = split * kSplitChunk, step = S * kSplitChunk;
-    const bool is_long = LPP == 16 && group > 1 && seq > kLongRounds * step;
+    const bool is_long = RING && group > 1 && seq > kLongRounds * step;
     // Long sequences: the chunks come through an LDS ring, loaded once a
     // workgroup by LDS DMA kLongStages - 1 chunks ahead.  DMA instruction j of a
     // chunk's 16 moves 4 rows of K (j < 8) or V; wave w issues j = w, w + group,
@@ -861,7 +864,7 @@ __global__ __launch_bounds__(512) void rf_attn_split_kernel(const float* __restr
                         store8_f16(qk.vc + c, vx);
                         typedef _Float16 hv8 __attribute__((ext_vector_type(8)));
                         hv8 hk, hvv;
-    #pragma unroll
+#pragma unroll
                         for (int i = 0; i < 8; ++i) {
                             hk[i] = (_Float16)kx[i];
                             hvv[i] = (_Float16)vx[i];
@@ -889,7 +892,6 @@ __global__ __launch_bounds__(512) void rf_attn_split_kernel(const float* __restr
             case 4: asm volatile("s_waitcnt vmcnt(%0)" :: "n"(4 * (kLongStages - 2)) : "memory"); break;
             case 6: asm volatile("s_waitcnt vmcnt(%0)" :: "n"(6 * (kLongStages - 2)) : "memory"); break;
             case 8: asm volatile("s_waitcnt vmcnt(%0)" :: "n"(8 * (kLongStages - 2)) : "memory"); break;
-            case 16: asm volatile("s_waitcnt vmcnt(%0)" :: "n"(16 * (kLongStages - 2)) : "memory"); break;
             default: asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
             }
             lds_barrier();
@@ -1216,17 +1218,27 @@ static hipError_t attn_decode(float* out, const float* q, const __half* kc, cons
         }
         const dim3 grid(nkv, S), blk(64 * group);
         const QkStep a = qk ? *qk : QkStep{};
-#define RF_SPLIT(LPP)                                                                                                  \
+        // the LDS ring only where its 16-byte DMA can read the caches (the per-lane
+        // loads take any address)
+        const bool ring = d == 128 &&
+                          ((reinterpret_cast<uintptr_t>(kc) | reinterpret_cast<uintptr_t>(vc)) & 15u) == 0;
+#define RF_SPLIT(LPP, RING)                                                                                            \
     if (qk)                                                                                                            \
-        hipLaunchKernelGGL((rf_attn_split_kernel<LPP, true>), grid, blk, 0, st, q, kc, vc, len_ptr, len, nh, nkv,      \
-                           scale, ws, S, a);                                                                           \
+        hipLaunchKernelGGL((rf_attn_split_kernel<LPP, true, RING>), grid, blk, 0, st, q, kc, vc, len_ptr, len, nh,     \
+                           nkv, scale, ws, S, a);                                                                      \
     else                                                                                                               \
-        hipLaunchKernelGGL((rf_attn_split_kernel<LPP, false>), grid, blk, 0, st, q, kc, vc, len_ptr, len, nh, nkv,     \
-                           scale, ws, S, a)
+        hipLaunchKernelGGL((rf_attn_split_kernel<LPP, false, RING>), grid, blk, 0, st, q, kc, vc, len_ptr, len, nh,    \
+                           nkv, scale, ws, S, a)
         switch (d) {
-        case 64: RF_SPLIT(8); break;
-        case 128: RF_SPLIT(16); break;
-        default: RF_SPLIT(32); break;
+        case 64: RF_SPLIT(8, false); break;
+        case 128:
+            if (ring) {
+                RF_SPLIT(16, true);
+            } else {
+                RF_SPLIT(16, false);
+            }
+            break;
+        default: RF_SPLIT(32, false); break;
         }
 #undef RF_SPLIT
         hipLaunchKernelGGL(rf_attn_merge_kernel, dim3(nh), dim3(256), 0, st, ws, out, nh, d, S);

@@ -74,3 +74,31 @@ def test_folded_step_gives_the_same(rf, dev, seq, nh, nkv):
     assert torch.equal(k.view(torch.int16), k2.view(torch.int16))
     assert torch.equal(v.view(torch.int16), v2.view(torch.int16))
     assert torch.equal(a, b) and bool(a.isfinite().all())
+
+
+@pytest.mark.parametrize("shift", [1, 2, 4, 8])      # halves: 2-, 4-, 8- and 16-byte addresses
+@pytest.mark.parametrize("seq,nh,nkv", [(6200, 8, 2), (7168, 16, 2), (600, 8, 2)])
+def test_caches_off_a_16_byte_address(rf, dev, seq, nh, nkv, shift):
+    # any address the cache's type allows, at every length
+    q, k, v = setup(seq, nh, nkv, seq + shift)
+    kb, vb = (torch.full((k.numel() + 8,), math.nan, dtype=torch.float16, device="cuda") for _ in range(2))
+    ks, vs = (b[shift:shift + k.numel()] for b in (kb, vb))
+    ks.copy_(k.view(-1))
+    vs.copy_(v.view(-1))
+    out, st = G.empty(nh * D, torch.float32), torch.tensor([seq - 1, seq], dtype=torch.int32, device="cuda")
+    ws, n = workspace(rf, nh)
+    scale = 1.0 / math.sqrt(D)
+    G.call(rf.rf_flash_attn_decode_state_ws, G.ptr(out), G.ptr(q), G.ptr(ks), G.ptr(vs),
+           ctypes.c_void_p(st.data_ptr() + 4), nh, nkv, D, scale, G.ptr(ws), n)
+    ref = reference(q, k, v)
+    assert (out.view(nh, D).double() - ref).abs().max().item() <= 1e-5 * ref.abs().max().item()
+    # the folded step writes the last row: raw q, k and v in, no norm
+    rk, rv, out2, q2 = torch.randn(nkv * D, device="cuda"), torch.randn(nkv * D, device="cuda"), out.clone(), q.clone()
+    G.call(rf.rf_attn_decode_qk_norm_rope_state, G.ptr(out2), G.ptr(q), G.ptr(rk), G.ptr(rv), None, None, G.ptr(ks),
+           G.ptr(vs), G.ptr(st), nh, nkv, D, 1e-6, 1e6, 1, None, None, None, scale, G.ptr(ws), n)
+    G.call(rf.rf_qk_norm_rope_kv_write_state, G.ptr(q2), G.ptr(rk), G.ptr(rv), None, None, G.ptr(k), G.ptr(v),
+           G.ptr(st), nh, nkv, D, 1e-6, 1e6, 1, None, None, None)
+    assert torch.equal(ks, k.view(-1)) and torch.equal(vs, v.view(-1))
+    assert bool(kb[:shift].isnan().all()) and bool(kb[shift + k.numel():].isnan().all())
+    ref = reference(q2, k, v)
+    assert (out2.view(nh, D).double() - ref).abs().max().item() <= 1e-5 * ref.abs().max().item()
