@@ -30,6 +30,7 @@
 // every lane.  No launcher allocates, frees or synchronises.
 #include <hip/hip_fp16.h>
 
+#include <climits>
 #include <mutex>
 
 
@@ -613,7 +614,12 @@ constexpr int kSplitChunk = 32;
 // 4096, two rounds, 14.1 / 14.5; with one head to a KV head the direct walk is
 // as fast (4500 positions 14.0 against 17.6).
 constexpr int kLongRounds = 3;
-constexpr int kLongStages = 4;
+// Three stages are 48 KB, so three workgroups fit a CU beside the tables and a
+// grid of a few more than two a CU (S is rounded up: 520 at 10, 20 or 40 KV heads)
+// stays one round.  Four stages leave two a CU and were no faster with one round
+// either (32 / 8 heads, 16200 positions 22.5 / 21.7 us; 40 / 20 65 / 42, of which
+// the second round is most).
+constexpr int kLongStages = 3;
 constexpr int kLongHalf = kSplitChunk * 256;    // a chunk's K (or V) rows at D = 128
 
 // QK: the decode step's per-head Q/K norm, RoPE and KV write are folded in
@@ -636,8 +642,12 @@ struct QkStep {
     const float2* cs;      // cos / sin table (rf_rope_cos_sin_kernel), or null
 };
 
-// RING: long sequences take the ring (its LDS is part of every launch of the
-// instance); its 16-byte DMA needs caches on 16-byte addresses.
+// RING: long sequences take the ring; its 16-byte DMA needs caches on 16-byte
+// addresses.  Its LDS is part of every launch of the instance, so what cannot be
+// long (one head to a KV head, a bound on the sequence below the line) takes the
+// other one (us before / after: 24 / 24 heads at 2048 positions 17.2 / 13.7, 10 / 10
+// at 5000 19.3 / 15.5, 80 / 40 at 600, 2048 and 16200 13.3 / 11.3, 28.1 / 19.1 and
+// 117 / 72).
 template <int LPP, bool QK, bool RING>
 __global__ __launch_bounds__(512) void rf_attn_split_kernel(const float* __restrict__ q,
                                                             const __half* kc,    // not restrict: QK writes a row
@@ -1218,9 +1228,10 @@ static hipError_t attn_decode(float* out, const float* q, const __half* kc, cons
         }
         const dim3 grid(nkv, S), blk(64 * group);
         const QkStep a = qk ? *qk : QkStep{};
-        // the LDS ring only where its 16-byte DMA can read the caches (the per-lane
-        // loads take any address)
-        const bool ring = d == 128 &&
+        // the LDS ring only where the sequence may become long and its 16-byte DMA can
+        // read the caches (the per-lane loads take any address)
+        const int bound = len_ptr == nullptr ? len : max_seq > 0 ? max_seq : INT_MAX;
+        const bool ring = d == 128 && group > 1 && bound > kLongRounds * S * kSplitChunk &&
                           ((reinterpret_cast<uintptr_t>(kc) | reinterpret_cast<uintptr_t>(vc)) & 15u) == 0;
 #define RF_SPLIT(LPP, RING)                                                                                            \
     if (qk)                                                                                                            \

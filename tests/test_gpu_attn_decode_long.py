@@ -102,3 +102,33 @@ def test_caches_off_a_16_byte_address(rf, dev, seq, nh, nkv, shift):
     assert bool(kb[:shift].isnan().all()) and bool(kb[shift + k.numel():].isnan().all())
     ref = reference(q2, k, v)
     assert (out2.view(nh, D).double() - ref).abs().max().item() <= 1e-5 * ref.abs().max().item()
+
+
+@pytest.mark.parametrize("group,seq", [(1, 4096), (2, 1024), (2, 4096), (2, 16384)])
+def test_a_grid_just_above_two_workgroups_a_cu(rf, dev, group, seq):
+    # the split count is rounded up, so with most KV head counts the grid is a few more
+    # than two workgroups a CU: they run beside the others, not in a round of their own
+    # (which took 1.4 to 1.6 times as long), so the time follows the work
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    times = []
+    for nkv in (cus // 2, cus // 2 + 1):             # 2 and 2 + 4 / CUs workgroups a CU
+        nh = nkv * group
+        q = torch.randn(nh, D, device="cuda")
+        k, v = (torch.randn(seq, nkv, D, device="cuda", dtype=torch.float16) for _ in range(2))
+        out, st = G.empty(nh * D, torch.float32), torch.tensor([seq - 1, seq], dtype=torch.int32, device="cuda")
+        ws, n = workspace(rf, nh)
+        best = math.inf
+        for _ in range(12):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            for _ in range(10):
+                rc = rf.rf_flash_attn_decode_state_ws(
+                    G.ptr(out), G.ptr(q), G.ptr(k), G.ptr(v), ctypes.c_void_p(st.data_ptr() + 4), nh, nkv, D,
+                    1.0 / math.sqrt(D), G.ptr(ws), n, G.stream())
+                assert rc == 0
+            b.record()
+            b.synchronize()
+            best = min(best, a.elapsed_time(b))
+        times.append(best)
+    print(f"group {group}, {seq} positions: {times[0] * 100:.1f} us, {times[1] * 100:.1f} us")
+    assert times[1] < 1.2 * times[0]
