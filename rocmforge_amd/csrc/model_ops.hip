@@ -987,8 +987,8 @@ __global__ __launch_bounds__(256) void rf_attn_merge_kernel(const float* __restr
         M = xor_max<32, 1>(M);
         const float f = lv > 0.0f ? expf(mv - M) : 0.0f;   // splits without positions count 0
         fs[t] = f;
-        float lt = f * lv;
-        lt = xor_sum64(lt);
+        // the butterfly's first step fused with the product (of the own term)
+        const float lt = xor_sum<16, 1>(__fmaf_rn(f, lv, lane_xor<32>(__fmul_rn(f, lv))));
         if (t == 0) lt_s = lt;
     }
     __syncthreads();

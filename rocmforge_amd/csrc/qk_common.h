@@ -164,8 +164,8 @@ __device__ __forceinline__ float sq8(const float4& a, const float4& b) {
 
 // v of lane ^ O (O = 1, 2, .., 32) by VALU exchanges, without the LDS round
 // trip of __shfl_xor: v_permlane32_swap / _16_swap for 32 and 16, DPP
-// row_ror:8 for 8, row_shl:4 / row_shr:4 selected by lane bit 2 for 4, quad
-// permutes for 2 and 1.
+// row_ror:8 for 8, row_shl:4 / row_shr:4 into the banks without / with lane
+// bit 2 for 4, quad permutes for 2 and 1.
 template <int O>
 __device__ __forceinline__ float lane_xor(float v) {
     static_assert(O == 1 || O == 2 || O == 4 || O == 8 || O == 16 || O == 32, "one lane bit");
@@ -181,30 +181,55 @@ __device__ __forceinline__ float lane_xor(float v) {
     } else if constexpr (O == 8) {
         return dpp_f<0x128>(v);
     } else if constexpr (O == 4) {
-        const float up = dpp_f<0x104>(v), dn = dpp_f<0x114>(v);
-        return (lane & 4) ? dn : up;
+        const int b = __float_as_int(v);
+        const int up = __builtin_amdgcn_update_dpp(b, b, 0x104, 0xF, 0x5, false);           // row_shl:4, banks 0, 2
+        return __int_as_float(__builtin_amdgcn_update_dpp(up, b, 0x114, 0xF, 0xA, false));  // row_shr:4, banks 1, 3
     } else {
         return dpp_f<O == 2 ? kQuadXor2 : kQuadXor1>(v);
     }
 }
 
-// The xor butterfly v += v[lane ^ o] for o = FROM, .., TO, halving or
+// One step of a butterfly with a commutative op: op(v, v of lane ^ O) with the
+// same bits, in fewer instructions than lane_xor where that can be had.  A swap
+// of v with itself leaves the pair in its two results on both lanes; where the
+// step for 8 came before (EQ8: lanes i and i ^ 8 hold the same bits), row_ror:4
+// serves for 4.  (With lane_xor's selects, long sequences of the decode attention,
+// which takes 4 or 5 steps a position, were 4-6 % slower than with __shfl_xor.)
+template <int O, bool EQ8, class Op>
+__device__ __forceinline__ float xor_step(float v, Op op) {
+    if constexpr (O == 32 || O == 16) {
+        const uint32_t b = __float_as_uint(v);
+        const auto r = [&] {
+            if constexpr (O == 32)
+                return __builtin_amdgcn_permlane32_swap(b, b, false, false);
+            else
+                return __builtin_amdgcn_permlane16_swap(b, b, false, false);
+        }();
+        return op(__uint_as_float(r[0]), __uint_as_float(r[1]));
+    } else if constexpr (O == 4 && EQ8) {
+        return op(v, dpp_f<0x124>(v));
+    } else {
+        return op(v, lane_xor<O>(v));
+    }
+}
+
+// The xor butterfly v = op(v, v[lane ^ o]) for o = FROM, .., TO, halving or
 // doubling from one to the next.
-template <int FROM, int TO>
-__device__ __forceinline__ float xor_sum(float v) {
-    v += lane_xor<FROM>(v);
+template <int FROM, int TO, bool EQ8 = false, class Op>
+__device__ __forceinline__ float xor_butterfly(float v, Op op) {
+    v = xor_step<FROM, EQ8>(v, op);
     if constexpr (FROM == TO)
         return v;
     else
-        return xor_sum<(FROM > TO ? FROM / 2 : FROM * 2), TO>(v);
+        return xor_butterfly<(FROM > TO ? FROM / 2 : FROM * 2), TO, FROM == 8>(v, op);
+}
+template <int FROM, int TO>
+__device__ __forceinline__ float xor_sum(float v) {
+    return xor_butterfly<FROM, TO>(v, [](float a, float b) { return a + b; });
 }
 template <int FROM, int TO>
 __device__ __forceinline__ float xor_max(float v) {
-    v = fmaxf(v, lane_xor<FROM>(v));
-    if constexpr (FROM == TO)
-        return v;
-    else
-        return xor_max<(FROM > TO ? FROM / 2 : FROM * 2), TO>(v);
+    return xor_butterfly<FROM, TO>(v, [](float a, float b) { return fmaxf(a, b); });
 }
 
 // o = 32, 16, .., 1: every lane ends with the same sum
