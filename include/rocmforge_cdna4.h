@@ -119,9 +119,9 @@ hipError_t wmma_gemm_q6_k_launch(const float* input, const void* weights_q6_k, f
  * caller whose producing kernel already rounded A to fp16 (bit patterns as
  * uint16_t, row-major [M][K]).  Same operand values as
  * wmma_gemm_q4_k_launch(fp32 A), so the same products; A is read at half
- * the bytes and not converted.  256 x 128 tiles where they fill more than
- * half the CUs (M = 512 at N = 14336; they need N % 128 == 0), else
- * 64- or 128-row x 64-column tiles with K split over the waves of a
+ * the bytes and not converted.  256 x 128 tiles from M = 192 on where they
+ * fill more than half the CUs (M = 512 at N = 14336; they need N % 128 == 0),
+ * else 64- to 256-row x 64-column tiles with K split over the waves of a
  * workgroup, and over workgroups (partials in the stream's slot, added in
  * split order) when the tiles leave half the CUs idle.  M % 64 == 0,
  * N % 64 == 0, K % 256 == 0, input and weights 16-byte aligned. */

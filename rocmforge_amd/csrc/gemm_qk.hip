@@ -11,8 +11,8 @@
 // accumulate / SwiGLU launchers below) round A to fp16 in a pass of their
 // own into library-owned device memory (the same values the reference's
 // __float2half gives) and run the fp16-activation tiles:
-//  * rf_gemm_q4k_f16a_kernel (Q4_K where 256 x 128 tiles fill more than half
-//    of the CUs): 4 waves, each weight dequantised once per 256 rows of A,
+//  * rf_gemm_q4k_f16a_kernel (Q4_K from 129 rows on where 256 x 128 tiles fill
+//    more than half of the CUs): 4 waves, each weight dequantised once per 256 rows of A,
 //    A and the weight ring by LDS DMA.
 //  * rf_gemm_q4k_f16s_kernel / rf_gemm_q4k_f16w_kernel (Q4_K otherwise) and
 //    rf_gemm_q6k_f16a_kernel (Q6_K from K = 768): 8 waves (16 on Q4_K's 64-row
@@ -3115,8 +3115,8 @@ static void reduce_for(bool acc, const float* G, const float* part, int S, int M
         launch_reduce<0>(part, S, M, N, D, nullptr, st);
 }
 
-// Q4_K on fp16 activations: 256 x 128 tiles (rf_gemm_q4k_f16a_kernel) where
-// they fill more than half the CUs, else the K-sliced tiles: eight waves
+// Q4_K on fp16 activations: 256 x 128 tiles (rf_gemm_q4k_f16a_kernel) from 129
+// rows on where they fill more than half the CUs, else the K-sliced tiles: eight waves
 // (rf_gemm_q4k_f16s_kernel) on 256 rows (from M =
 // kQ4TallMinM: each weight dequantised once per 256 rows) or 128, sixteen
 // (rf_gemm_q4k_f16w_kernel) on 64 (M <= 64,
@@ -3165,7 +3165,11 @@ static hipError_t gemm_q4_f16(const uint16_t* A, const void* W, float* D, int M,
     // 160, 164 / 123; 1280 x 3840 x 2560, 150, 54 / 38; 1088 x 3584 x 18944,
     // 140, 280 / 209).  Accumulating (the old contents of a row block read ahead
     // of its stores) 2048 x 4096 x 12288 263 / 215, 2048 x 4096 x 4096 101 / 76.
-    if (2 * big > (long)device_cu_count()) {
+    // Up to 128 rows they would multiply nothing in half of the tile or more: 64 and
+    // 128 rows x 18944 x 3584 32.1 and 41.4 on the 64- and 128-row tiles against 49.7
+    // and 47.8, x 32768 34 and 49 against 60 and 63; 192 rows x 18944 60.8 / 49.4,
+    // x 32768 89.7 / 65.2; 320 x 8320 63.4 / 45.8.
+    if (M > 128 && 2 * big > (long)device_cu_count()) {
         if constexpr (ACC)
             hipLaunchKernelGGL(rf_gemm_q4k_f16a_kernel<4>, dim3((unsigned)big), dim3(kF16aThreads), 0, st, A, w, w, D,
                                M, N, K, nullptr, KSplit{1, nullptr});
@@ -3462,8 +3466,8 @@ extern "C" hipError_t rf_gemm_q6_k_f16_accumulate_launch(const uint16_t* input_f
     return q6_f16_checked<true>(input_f16, weights_q6_k, inout, M, N, K, stream);
 }
 
-// inout[M x N] += the product of rf_gemm_q4_k_f16_launch, on the K-sliced
-// tiles (each output read and written once after its fp32 sum).
+// inout[M x N] += the product of rf_gemm_q4_k_f16_launch, on the same tiles
+// (each output read and written once after its fp32 sum).
 extern "C" hipError_t rf_gemm_q4_k_f16_accumulate_launch(const uint16_t* input_f16, const void* weights_q4_k,
                                                          float* inout, int M, int N, int K, hipStream_t stream) {
     if (input_f16 == nullptr || weights_q4_k == nullptr || inout == nullptr) return hipErrorInvalidValue;
