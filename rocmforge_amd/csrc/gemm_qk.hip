@@ -15,8 +15,8 @@
 //    more than half of the CUs): 4 waves, each weight dequantised once per 256 rows of A,
 //    A and the weight ring by LDS DMA.
 //  * rf_gemm_q4k_f16s_kernel / rf_gemm_q4k_f16w_kernel (Q4_K otherwise) and
-//    rf_gemm_q6k_f16a_kernel (Q6_K from K = 768): 8 waves (16 on Q4_K's 64-row
-//    tiles) over 64- to 256-row x 64-column tiles, K
+//    rf_gemm_q6k_f16a_kernel (Q6_K from K = 768): 8 waves (mostly 16 on Q4_K's
+//    64-row tiles) over 64- to 256-row x 64-column tiles, K
 //    sliced over waves and added through LDS; when the tiles leave at least
 //    half the CUs idle, K is also split over workgroups whose partial tiles
 //    rf_gemm_split_reduce_kernel adds in split order.
@@ -2274,7 +2274,7 @@ constexpr int kQ4sThreads = 512;
 constexpr int kQ4sBN = 64;
 constexpr int kQ4sStage = 16 * 1024;                  // 64 rows x 144 B (+ padding DMAs)
 
-// FMR = 4 (128 rows) or 8.
+// FMR = 2 (64 rows, short ranges of a K split), 4 (128) or 8.
 // FMR = 8 (256 x 64 tiles): each weight dequantised once per 256 rows of A;
 // LDS then holds two ring stages and four 32 KB A buffers (one chunk of DMA
 // slack), as in the tall Q6_K tiles, and the K-slice partials go through
@@ -2528,7 +2528,8 @@ __device__ __forceinline__ void q4s_wg(const uint16_t* __restrict__ A, const uin
 
 // ── q4w: Q4_K GEMM on fp16 activations, 64 x 64 tiles on sixteen waves ────
 // (rf_gemm_q4_k_f16_launch and the launchers on it at M <= 64, and where
-// 64-row tiles come to at most one round of CUs).  A 64-row tile feeds each
+// 64-row tiles come to at most one round of CUs, but for short ranges of a
+// K split: q4_f16_tiles).  A 64-row tile feeds each
 // weight to two MFMAs only, so the wave's own instruction stream (about 70
 // per 64-wide chunk: dequantisation, scales, addresses, DMA issue) and its
 // waits set the time, not a unit: with the eight waves of
@@ -3118,9 +3119,9 @@ static void reduce_for(bool acc, const float* G, const float* part, int S, int M
 // Q4_K on fp16 activations: 256 x 128 tiles (rf_gemm_q4k_f16a_kernel) from 129
 // rows on where they fill more than half the CUs, else the K-sliced tiles: eight waves
 // (rf_gemm_q4k_f16s_kernel) on 256 rows (from M =
-// kQ4TallMinM: each weight dequantised once per 256 rows) or 128, sixteen
-// (rf_gemm_q4k_f16w_kernel) on 64 (M <= 64,
-// or when they come to at most one round of CUs), split over K when
+// kQ4TallMinM: each weight dequantised once per 256 rows), 128, or 64 (M <= 64,
+// or when they come to at most one round of CUs; there mostly sixteen waves,
+// rf_gemm_q4k_f16w_kernel), split over K when
 // they leave at least half the CUs idle and `part` is given.
 // G: when given, D receives fp16 silu(G) * (A W^T) (the up projection of a
 // SwiGLU whose gate product G [M x N] is already computed)
@@ -3135,12 +3136,22 @@ static void q4_f16_tiles(const uint16_t* A, const uint8_t* w, float* D, int M, i
                          const float* G, const PartBuf& part, const RowNorm* rn = nullptr) {
     const long tiles = (long)((M + 32 * FMR - 1) / (32 * FMR)) * (N / kQ4sBN);
     const int S = 2 * tiles <= (long)device_cu_count() ? ksplit_count(tiles, K / kQK, M, N, part) : 1;
+    // 64-row tiles split over K: sixteen waves where a workgroup's range is long enough
+    // to pay for filling their deeper pipeline and for adding eight partials in place
+    // of four (us, eight / sixteen waves, super-blocks a workgroup in brackets:
+    // 64 x 512 x 1024 [1] 9.1 / 9.5, 192 x 512 x 2560 [1] 11.2 / 12.0, 64 x 512 x 4096
+    // [2] 11.3 / 11.7, [3] 1-2 % slower, [4] alike, from [5] on 2-10 % faster; with more
+    // than 1024 rows A's traffic counts, 2048 x 256 x 2560 [5] 14.9 / 15.4, [8] alike).
+    // Unsplit always: storing they lose 1-3 % at one or two super-blocks and on
+    // 2048 x 512 up to K = 2560 (13.4 / 13.9 at 1536), accumulating, which takes the
+    // same tiles for the same bits, they gain 12-25 % there, and elsewhere both gain.
+    auto wide16 = [&](int S) { return FMR == 2 && (S == 1 || K / kQK / S >= (M > 1024 ? 8 : 5)); };
     auto go = [&](auto accc, float* d, const float* g, const KSplit& sp) {
         constexpr bool kAcc = decltype(accc)::value;
         const dim3 grid((unsigned)(tiles * sp.S));
-        if constexpr (FMR == 2)
+        if (wide16(sp.S))
             hipLaunchKernelGGL(rf_gemm_q4k_f16w_kernel<kAcc>, grid, dim3(kQ4wThreads), 0, st, A, w, d, M, N, K, g, sp);
-        else
+        else if constexpr (!(kAcc && FMR == 2))      // (64 rows accumulate unsplit, above)
             hipLaunchKernelGGL((rf_gemm_q4k_f16s_kernel<FMR, kAcc>), grid, dim3(kQ4sThreads), 0, st, A, w, d, M, N, K,
                                g, sp);
     };

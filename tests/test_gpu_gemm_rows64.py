@@ -47,3 +47,26 @@ def test_store_accumulate_and_swiglu(rf, dev, m, n, k):
     ref = O.gemm("q4_k", a, w, m, n, k)
     tol = 2e-3 * np.abs(ref) + 2e-5 * O.gemm_abs("q4_k", a, w, m, n, k)     # the GEMM bar
     assert (np.abs(got - ref) <= tol).all()
+
+
+# Short ranges of a K split stay on eight waves with four K slices, as the segment
+# launcher's tiles take them: its products of the ranges, added in order, have the
+# same bits (these few tiles are split into single super-blocks, or pairs)
+@pytest.mark.parametrize("m,n,k,split", [(64, 64, 512, 2), (64, 192, 768, 3), (128, 64, 1024, 4), (64, 128, 4096, 8)])
+def test_short_k_ranges_on_eight_waves(rf, dev, m, n, k, split):
+    a = synth.activations(k, seed=m + n, m=m).astype(np.float16)
+    w = synth.weights("q4_k", n, k, seed=k).reshape(n, k // 256, -1)
+    z = None
+    want, part = None, G.empty(m * n, torch.float32)
+    for s in range(split):
+        ks = slice(s * k // split, (s + 1) * k // split)
+        da = G.to_dev(np.ascontiguousarray(a[:, ks]).view(np.int16))
+        dw = G.to_dev(np.ascontiguousarray(w[:, ks.start // 256:ks.stop // 256]))
+        G.call(rf.rf_gemm_qk_f16_segments_launch, G.ptr(da), G.ptr(dw), z, z, 12, 12, 12, G.ptr(part), z, z, m, n, 0,
+               0, k // split)
+        got = G.host(part).reshape(m, n)
+        want = got if want is None else want + got
+    d = G.empty(m * n, torch.float32)
+    da, dw = G.to_dev(a.view(np.int16)), G.to_dev(w.reshape(-1))
+    G.call(rf.rf_gemm_q4_k_f16_launch, G.ptr(da), G.ptr(dw), G.ptr(d), m, n, k)
+    np.testing.assert_array_equal(G.host(d).reshape(m, n), want)
