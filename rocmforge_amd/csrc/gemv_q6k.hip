@@ -290,8 +290,7 @@ __global__ __launch_bounds__(512) void rf_q6k_gemv_xreg_kernel(const uint8_t* __
         }
         float t0, t1;
         q6_dot16x2(v0, xr[0], v1, xr[1], t0, t1);
-        float acc = s0 * (t0 - 32.0f * xs[0]);
-        acc += s1 * (t1 - 32.0f * xs[1]);
+        const float acc = q6_lane_term(s0, t0, xs[0], s1, t1, xs[1]);
         const float tot = wave_sum(live ? acc : 0.0f);
         if (lane == 0) part[j * nwk + wave] = tot;
     };
@@ -334,13 +333,12 @@ __global__ __launch_bounds__(512) void rf_q6k_gemv_lin_kernel(const uint8_t* __r
 template <int NB, int MAXW>
 __global__ __launch_bounds__(64 * MAXW) void rf_q6k_gemv_any_kernel(const uint8_t* __restrict__ w,
                                                                     const float* __restrict__ x,
-                                                                    const float* residual, float* y, int K, int N,
-                                                                    int gk) {
+                                                                    const float* residual, float* y, int K, int N) {
     __shared__ __align__(16) uint8_t stage_lds[MAXW * 2048];
     extern __shared__ __align__(16) float part[];   // [rows of this workgroup][NWK][4 lane rows]
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     q6_lin_team<NB, true>(w, x, residual, y, K, N, nullptr, 1.0f, blockIdx.x, gridDim.x, wave, blockDim.x / kWave,
-                          stage_lds + wave * 2048, part, gk);
+                          stage_lds + wave * 2048, part);
 }
 
 }  // namespace rf
@@ -381,10 +379,10 @@ static hipError_t launch_q6(const void* weights_q6_k, const float* input, const 
         if (lds + (nwk <= 8 ? 8 : 16) * 2048 <= 64 * 1024) {
             if (nwk <= 8)
                 hipLaunchKernelGGL((rf_q6k_gemv_any_kernel<kQ6Ring, 8>), dim3(grid), dim3(nwk * 64), lds, stream, w,
-                                   input, residual, output, n_rows, ncols_dst, gk);
+                                   input, residual, output, n_rows, ncols_dst);
             else
                 hipLaunchKernelGGL((rf_q6k_gemv_any_kernel<kQ6Ring, 16>), dim3(grid), dim3(nwk * 64), lds, stream, w,
-                                   input, residual, output, n_rows, ncols_dst, gk);
+                                   input, residual, output, n_rows, ncols_dst);
             return hipGetLastError();
         }
     }

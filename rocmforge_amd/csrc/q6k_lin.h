@@ -83,19 +83,25 @@ __device__ __forceinline__ void q6_x_prep(float (&xr)[2][16], float (&xs)[2]) {
 // is one row, and 8 rows are a multiple of 16 bytes.  The matrix is 16-byte
 // aligned, so only its last piece can reach past its end: that one is read at
 // the matrix's last 16 bytes and shifted into place.  Row sums are then
-// grouped per wave, ((r0 + r1) + (r2 + r3)) in team-wave order, and which of a
-// lane's two products is rounded before the fma follows the row's place in the
-// ring: the bits that rf_q6k_gemv_xreg_kernel, which takes any 2-byte aligned
-// matrix, compiles to (a decode step's 8-bit inputs turn a last-bit change into
-// one of 1e-3, so a layer's kernels keep theirs).
+// grouped per wave, ((r0 + r1) + (r2 + r3)) in team-wave order: the bits of
+// rf_q6k_gemv_xreg_kernel, which takes any 2-byte aligned matrix.
 //
 // Row j's sum is the team's 4 nwk partial sums (16-lane row sums, in
-// team-wave order) added in that order, whatever the grid.  Every thread of
+// team-wave order) added in that order (ANY: grouped as above), whatever the
+// grid.  Every thread of
 // the workgroup calls this once (one barrier before the final sums); part
 // holds nrows * nwk * 4 floats of this team.
 struct Q6Seg {
     u32x4 a, b;
 };
+
+// A lane's part of a row: its two 16-weight runs, scales s, dots t of the raw
+// quants, sums xs of x.  The roundings are spelled out, so that every kernel that
+// calls this gives the same bits.
+__device__ __forceinline__ float q6_lane_term(float s0, float t0, float xs0, float s1, float t1, float xs1) {
+    const float u0 = __builtin_fmaf(-32.0f, xs0, t0), u1 = __builtin_fmaf(-32.0f, xs1, t1);
+    return __builtin_fmaf(s1, u1, __fmul_rn(s0, u0));
+}
 typedef uint32_t u32x4a2 __attribute__((ext_vector_type(4), aligned(2)));
 
 // v shifted down by `bytes` (even, 0..14, the same in all lanes)
@@ -112,7 +118,7 @@ template <int NB, bool ANY = false>
 __device__ __forceinline__ void q6_lin_team(const uint8_t* __restrict__ w, const float* __restrict__ x,
                                             const float* residual, float* y, int K, int N,
                                             const float* __restrict__ norm_w, float inv, int g, int G, int tw,
-                                            int nwk, uint8_t* stage, float* part, int gk = 1) {
+                                            int nwk, uint8_t* stage, float* part) {
     const int lane = threadIdx.x & (kWave - 1);
     const int nsb = K / kQK;
     const size_t row_bytes = (size_t)nsb * kQ6KBytes;
@@ -148,11 +154,6 @@ __device__ __forceinline__ void q6_lin_team(const uint8_t* __restrict__ w, const
     // chunks past the last re-read it (same line), written to the spare area
     const int c0 = ANY ? min(lane, last) : lane, c1 = min(64 + lane, last);
     const int over = ANY ? (int)(0u - (uint32_t)((size_t)N * row_bytes)) & 15 : 0;   // of the matrix's last piece
-    // row j is row j0 + gk j of the G / gk workgroups the association refers to,
-    // of whose nr0 rows the first ring_rows are in the pipeline's full rounds
-    const int g0 = ANY ? G / gk : 1, j0 = ANY ? g / g0 : 0;
-    const int nr0 = g < N ? (N - 1 - (g - j0 * g0)) / g0 + 1 : 0;
-    const int ring_rows = nr0 < NB ? 0 : nr0 / NB * NB;
     const bool tail = ANY && over && 8 * tw + nblk == nsb;
     auto load = [&](Q6Seg& u, int j) {
         const int row = nrows ? g + min(j, nrows - 1) * G : 0;
@@ -225,10 +226,7 @@ __device__ __forceinline__ void q6_lin_team(const uint8_t* __restrict__ w, const
         q6_dot16x2(v0, xr[0], v1, xr[1], t0, t1);
         float acc;
         if constexpr (ANY) {
-            const float u0 = t0 - 32.0f * xs[0], u1 = t1 - 32.0f * xs[1];
-            const float f0 = __builtin_fmaf(s0, u0, __fmul_rn(s1, u1)), f1 = __builtin_fmaf(s1, u1, __fmul_rn(s0, u0));
-            const int jr = j0 + gk * j;
-            acc = jr % NB != 0 && jr < ring_rows ? f0 : f1;
+            acc = q6_lane_term(s0, t0, xs[0], s1, t1, xs[1]);
         } else {
             acc = s0 * (t0 - 32.0f * xs[0]);
             acc += s1 * (t1 - 32.0f * xs[1]);

@@ -42,3 +42,18 @@ def test_same_bits_as_a_matrix_off_a_16_byte_address(rf, dev, k, n):
     G.call(rf.gemv_q6_k_f32_launch, G.ptr(dw), G.ptr(dx), G.ptr(a), k, n)
     G.call(rf.gemv_q6_k_f32_launch, G.ptr(raw[2:]), G.ptr(dx), G.ptr(b), k, n)
     np.testing.assert_array_equal(G.host(a), G.host(b))
+
+
+# rows per workgroup from one to several rounds of the pipeline; a second N moves the
+# rows to other places of it, an address off 16 bytes to the kernel with direct loads
+@pytest.mark.parametrize("k,n", [(1280, 9001), (2560, 4099), (3584, 12007), (11008, 3001), (16128, 1999)])
+def test_a_row_gives_the_same_bits_in_any_place(rf, dev, k, n):
+    row, x = synth.weights("q6_k", 8, k, seed=k).reshape(8, -1)[3], synth.activations(k, seed=n)
+    dw, dx = G.to_dev(np.tile(row, n)), G.to_dev(x)
+    off = G.to_dev(np.concatenate([np.zeros(2, np.uint8), np.tile(row, n)]))
+    want = None
+    for w, rows in ((dw, n), (dw, n - 777), (dw, 64), (off[2:], n), (off[2:], n - 777)):
+        y = G.empty(rows, torch.float32)
+        G.call(rf.gemv_q6_k_f32_launch, G.ptr(w), G.ptr(dx), G.ptr(y), k, rows)
+        want = y[0].item() if want is None else want
+        assert bool((y == want).all())
