@@ -14,9 +14,11 @@
 //    matrix.  K split across the waves of a workgroup (8 super-blocks per
 //    wave), x held in registers, weights read with lane-linear aligned
 //    16-byte loads and restaged per wave through LDS.
-//  * rf_q6k_gemv_any_kernel: K <= 32768 otherwise, 16-byte aligned matrix.
+//  * rf_q6k_gemv_any_kernel: K <= 32768 otherwise, 16-byte aligned matrix
+//    (up to K = 8192 from some hundred or thousand rows on: launch_q6).
 //    The same, with rows that start anywhere in a 16-byte piece.
-//  * rf_q6k_gemv_xreg_kernel: K <= 16384, matrices off a 16-byte address.
+//  * rf_q6k_gemv_xreg_kernel: K <= 16384, few rows or a matrix off a 16-byte
+//    address.
 //    Same K split and x registers, each lane loading its block fields
 //    directly (16-byte loads at the 2-byte aligned block offsets).
 //  * rf_q6k_gemv_kernel: the rest.  One row per wave step, four lanes per
@@ -362,18 +364,30 @@ static hipError_t launch_q6(const void* weights_q6_k, const float* input, const 
             return hipGetLastError();
         }
     }
-    // below a megabyte the launch is a row or two a wave and its latency counts:
-    // the direct loads are quicker (512 x 1280 2.84 against 3.01 us, 129 x 1792
-    // 2.6 against 2.8; 1001 x 2304, 1.9 MB, 4.29 against 3.88)
-    if (nsb <= 128 && (reinterpret_cast<uintptr_t>(w) & 15u) == 0 &&
-        (nsb > 64 || (size_t)ncols_dst * nsb * kQ6KBytes >= (1u << 20))) {
-        const int nwk = (nsb + 7) / 8;
-        // a multiple of 8, so that the rows of a workgroup share their phase;
-        // with two to seven slices twice the workgroups are faster (151936 x 2560
-        // 80 against 89 us, 4096 x 11008 11.8 against 12.3; one slice 121971 x
-        // 1536 45 against 39, ten 3584 x 18944 17.2 against 15.0)
-        const int cap = std::max(device_cu_count() * (nwk >= 4 ? 1 : 8 / nwk) / 8 * 8, 8);
-        const int gk = ncols_dst > cap && nwk >= 2 && nwk <= 7 ? 2 : 1;
+    // Rows a CU from which the lane-linear kernel is the faster one, and from which it
+    // takes twice the workgroups, by the number of K slices.  Below, a wave has a row or
+    // two and the direct loads' shorter way counts; with four slices its one workgroup a
+    // CU has too few loads in flight.  Speed against the direct loads with one / twice the
+    // workgroups (rows x K, weights from HBM; in brackets from the Infinity Cache):
+    //   one slice     1024 x 1280 1.00 / 1.00 (0.98), 1280 1.06, 32000 1.34 / 1.10
+    //   two           512 x 3072 1.03, 1536 x 3840 1.09 / 0.84, 12288 x 3840 1.28 / 1.17,
+    //                 16384 x 2304 1.33 / 1.41 and x 3840 1.27 / 1.26, 152064 x 3072 1.34 / 1.53
+    //   three         512 x 5888 1.05, 2560 1.08 / 1.00 (1.04 / 1.10), 3584 1.10 / 1.06
+    //                 (1.02 / 1.12), 4608 x 4352 1.19 / 1.30
+    //   four          2048 x 7168 0.97 / 0.99, 2560 0.95 / 1.02 (0.88 / 1.03), 32000 0.91 / 1.31
+    //   five          512 x 9984 1.04 / 0.93, 1536 x 8448 1.03 / 1.03 (0.99 / 1.09)
+    //   six           512 x 12032 1.04 / 0.88, 4096 1.12 / 1.09 (1.03 / 1.07), 8192 1.17 / 1.19
+    //   seven         512 x 14080 1.05 / 0.86, 8192 1.23 / 1.22 (1.00 / 1.02), 12288 1.22 / 1.26
+    //   eight         512 x 16128 1.07 / 0.85, 4096 1.26 / 1.20
+    constexpr int kNever = 1 << 20;
+    constexpr int kLinFrom[9] = {0, 5, 2, 2, 10, 0, 0, 0, 0};
+    constexpr int kTwiceFrom[9] = {0, kNever, 64, 14, 10, 6, 16, 32, kNever};
+    const long cus = device_cu_count();
+    const int nwk = (nsb + 7) / 8;
+    if (nsb <= 128 && (reinterpret_cast<uintptr_t>(w) & 15u) == 0 && (nwk > 8 || ncols_dst >= kLinFrom[nwk] * cus)) {
+        // a multiple of 8, so that the rows of a workgroup share their phase
+        const int cap = (int)std::max(cus * (nwk >= 4 ? 1 : 8 / nwk) / 8 * 8, 8L);
+        const int gk = nwk <= 8 && ncols_dst >= kTwiceFrom[nwk] * cus ? 2 : 1;
         const int grid = ncols_dst < cap ? ncols_dst : cap * gk;
         const size_t lds = (size_t)((ncols_dst + grid - 1) / grid) * nwk * 4 * sizeof(float);
         if (lds + (nwk <= 8 ? 8 : 16) * 2048 <= 64 * 1024) {
@@ -387,7 +401,6 @@ static hipError_t launch_q6(const void* weights_q6_k, const float* input, const 
         }
     }
     if (nsb <= 64) {
-        const int nwk = (nsb + 7) / 8;
         // about 8 waves per CU: short K (few slices per workgroup) gets
         // several workgroups per CU
         const int cap = device_cu_count() * (nwk >= 4 ? 1 : 8 / nwk);

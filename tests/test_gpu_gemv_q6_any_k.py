@@ -57,3 +57,22 @@ def test_a_row_gives_the_same_bits_in_any_place(rf, dev, k, n):
         G.call(rf.gemv_q6_k_f32_launch, G.ptr(w), G.ptr(dx), G.ptr(y), k, rows)
         want = y[0].item() if want is None else want
         assert bool((y == want).all())
+
+
+# on both sides of the lines in rows (256 CUs): one slice 1280; two 512, 16384; three
+# 512, 3584; four 2560; five 1536; six 4096; seven 8192
+@pytest.mark.parametrize("k,n", [(1792, 1280), (2304, 512), (2304, 16384), (5888, 512), (5888, 3584), (7424, 2560),
+                                 (8448, 1536), (12032, 4096), (13824, 8192)])
+def test_both_sides_of_the_lines_in_rows(rf, dev, k, n):
+    w, x = synth.weights("q6_k", 256, k, seed=k + 1), synth.activations(k, seed=k + 2)
+    w = np.tile(w.reshape(256, -1), (-(-n // 256), 1))[:n].reshape(-1)
+    raw = G.to_dev(np.concatenate([np.zeros(2, np.uint8), w]))
+    dw, dx = G.to_dev(w), G.to_dev(x)
+    ref = O.gemv_q6k(w[:256 * (k // 256) * 210], x, k, 256)
+    for rows in (n, n - 1):
+        a, b = G.empty(rows, torch.float32), G.empty(rows, torch.float32)
+        G.call(rf.gemv_q6_k_f32_launch, G.ptr(dw), G.ptr(dx), G.ptr(a), k, rows)
+        G.call(rf.gemv_q6_k_f32_launch, G.ptr(raw[2:]), G.ptr(dx), G.ptr(b), k, rows)
+        np.testing.assert_array_equal(G.host(a), G.host(b))
+        rel, worst = G.gemv_error(G.host(a)[-512:], np.tile(ref, -(-rows // 256))[:rows][-512:])
+        assert rel <= 1e-5 and worst <= 1.0, (rel, worst)
