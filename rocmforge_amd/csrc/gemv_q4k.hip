@@ -732,17 +732,25 @@ static hipError_t launch_q4_lin(const void* w, const float* x, const float* res,
 }
 
 // Other K above 8192 where the one-row-per-step kernel's last step, two rows for
-// each of its 4 CUs waves, leaves at least an eighth of all its row slots empty
-// (rf_q4k_q8_any_kernel, the same bits; figures there).  With the slots full it
-// is the slower one from three slices of K up (us, row steps / this: 4096 x
-// 11008 9.0 / 9.4, 8192 x 18944 20.6 / 22.0), and with two slices it has too few
-// waves (2560 x 6912 6.0 / 6.8, 4096 x 5120 6.2 / 8.2).  false: not launched.
+// each of its 4 CUs waves, leaves enough of all its row slots empty
+// (rf_q4k_q8_any_kernel, the same bits; figures there).  Speed of this kernel against
+// the row steps by the share of the slots filled, weights from HBM (in brackets
+// from the Infinity Cache), 256 CUs:
+//   three slices (K to 12288)  1536 rows, 3/4: 1.10 (1.04); 3072, 3/4: 1.16 (1.10);
+//                              3276, 0.8: 1.03 (0.97); 3584, 7/8: 1.00 (0.95)
+//   four and more, one step    1536 rows, 3/4: 1.02-1.07 (0.98-1.13); 1792, 7/8: 0.99-1.05 (0.95-1.07)
+//   two steps                  3584 rows, 7/8: 1.04-1.11 (1.05-1.14); 3850, 0.94: 0.99-1.08 (0.99-1.10)
+//   three and four             5120 x 13824, 5/6: 12.9 / 12.2 us, 5120 x 27648 21.7 / 19.6; 6881 rows,
+//                              0.84: 1.00-1.13 (0.97-1.15); 7372, 0.9: 0.96-1.09 (0.94-1.09)
+// and with two slices it has too few waves (2560 x 6912 6.0 / 6.8 us, 4096 x 5120
+// 6.2 / 8.2).  false: not launched.
 static bool launch_q4_any(const void* w, const float* x, const float* res, float* y, int K, int N, hipStream_t st,
                           hipError_t* e) {
     const int cap = device_cu_count();
-    const long step = 8L * cap, slots = (N + step - 1) / step * step;
-    if (K <= 8192 || !aligned16(x) || 8L * N > 7 * slots) return false;
     const int nwk = (K + 4095) / 4096;
+    const long step = 8L * cap, steps = (N + step - 1) / step, slots = steps * step;
+    const bool gaps = nwk == 3 || steps == 1 ? 4L * N <= 3 * slots : steps == 2 ? 8L * N <= 7 * slots : 6L * N <= 5 * slots;
+    if (K <= 8192 || !aligned16(x) || !gaps) return false;
     const int grid = N < cap ? N : cap;
     const size_t lds = ((size_t)((N + grid - 1) / grid) + 1) * nwk * kWave * sizeof(float2);
     if (lds > 160 * 1024) return false;

@@ -39,3 +39,19 @@ def test_bits_of_the_row_step_kernel(rf, dev, n, k):
     inout = dr[:n].clone()
     G.call(rf.gemv_q4_k_f32_q8_inline_residual_launch, G.ptr(dw), G.ptr(dx), G.ptr(inout), G.ptr(inout), k, n)
     assert torch.equal(inout, got[:n])
+
+
+# the fullest the kernel takes (256 CUs: 2048 rows a step of the other kernel), by
+# steps and slices of K, against the same rows of a matrix that fills the steps
+@pytest.mark.parametrize("n,k", [(1536, 8448), (3072, 11008), (1536, 13824), (3584, 18944), (5120, 13824)])
+def test_at_the_lines(rf, dev, n, k):
+    step = 8 * torch.cuda.get_device_properties(0).multi_processor_count
+    full = -(-n // step) * step
+    part = synth.weights("q4_k", 512, k, seed=k).reshape(512, -1)
+    w, x = part.repeat(-(-full // 512), axis=0)[:full].reshape(-1), synth.activations(k, seed=n)
+    dw, dx = G.to_dev(w), G.to_dev(x)
+    ref, got = G.empty(full, torch.float32), G.empty(n, torch.float32)
+    f = rf.gemv_q4_k_f32_q8_inline_launch
+    G.call(f, G.ptr(dw), G.ptr(dx), G.ptr(ref), k, full)
+    G.call(f, G.ptr(dw), G.ptr(dx), G.ptr(got), k, n)
+    assert torch.equal(got, ref[:n])
