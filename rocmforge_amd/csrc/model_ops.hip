@@ -2158,17 +2158,22 @@ static hipError_t attn_prefill(const void* Q, const void* K, const void* V, OUT*
     if ((reinterpret_cast<uintptr_t>(Q) | reinterpret_cast<uintptr_t>(K) | reinterpret_cast<uintptr_t>(V)) & 15u)
         return hipErrorInvalidValue;
     // 32-query units over the CUs (64 KB of LDS per key group, so at most two
-    // workgroups on a CU): two units and two key groups a workgroup while those
-    // workgroups are one a CU or fewer (512 positions, 32 heads: 10.5 us, four
-    // units 13.5, eight units unsplit 19.2), eight unsplit units where they come
-    // to two a CU, so that long and short query blocks even out (4096 positions:
-    // 143 us against 157 with four units and two key groups), four units and two
-    // key groups between (2048: 47 against 61 and 57; these figures from one run
-    // of a form with a cheaper rescale, all routes alike)
+    // workgroups of one group on a CU).  Causal: two units and two key groups a
+    // workgroup up to three units a CU, eight unsplit units from eleven on, where long
+    // and short query blocks even out, four units and two key groups between.  us,
+    // two / four / eight units, 32 / 8 heads unless named: 576 units 12.9 / 16.3 / 22.3,
+    // 768 16.7 / 19.1 / 27.4 (64 / 8 heads 13.7 / 13.4), 1024 22.7 / 23.3 / 34 (64 / 8
+    // 17.0 / 15.8), 1152 30.1 / 25.4 / 37; 2560 98 / 81.8 / 83.3, 2816 114 / 94.3 / 93.0 (64 / 8
+    // 74 / 59 / 52), 3584 175 / 134 / 120, 4032 216 / 165 / 147.  Without a mask all units are
+    // equally long and whole rounds count: two units up to two a CU, then four or
+    // eight by their rounds, one of eight taking about 1.6 of four's (1152 units 50 /
+    // 48 / 37.8, 2048 110 / 85.5 / 79.2, 2304 147 / 130 / 149, 3072 228 / 178 / 196, 3584 304 /
+    // 257 / 228).
     const long long units = (long long)num_q_heads * (seq_len / 32), cus = rf::device_cu_count();
-    if (units <= 2 * cus)
+    const long long rounds4 = (units + 4 * cus - 1) / (4 * cus), rounds8 = (units + 8 * cus - 1) / (8 * cus);
+    if (units <= (causal ? 3 : 2) * cus)
         attn_prefill_go<4, 2, true>(Q, K, V, O, seq_len, num_q_heads, num_kv_heads, causal, scale, stream);
-    else if (units < 16 * cus)
+    else if (causal ? units < 11 * cus : 8 * rounds8 > 5 * rounds4)
         attn_prefill_go<8, 2, false>(Q, K, V, O, seq_len, num_q_heads, num_kv_heads, causal, scale, stream);
     else
         attn_prefill_go<8, 1, true>(Q, K, V, O, seq_len, num_q_heads, num_kv_heads, causal, scale, stream);

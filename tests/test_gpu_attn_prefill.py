@@ -119,3 +119,16 @@ def test_large_scores(rf, dev, seq, nq, nkv, size, sign):
     group = nq // nkv
     bound = 1e-3 * U16 * mag[:, :group] + 1e-6
     assert bool(((got - ref)[:, :group].abs() <= bound)[clear].all())
+
+
+# both sides of the lines between the routes (256 CUs): causal 768 and 2816 units of 32
+# queries, without a mask 512, 1024, 2048 and 3072
+@pytest.mark.parametrize("seq,nq,nkv,causal", [(768, 32, 8, 1), (832, 32, 8, 1), (1024, 88, 8, 1), (960, 90, 9, 1),
+                                               (512, 32, 8, 0), (576, 32, 8, 0), (1024, 32, 8, 0), (1088, 32, 8, 0),
+                                               (2048, 32, 8, 0), (2112, 32, 8, 0), (3136, 32, 8, 0)])
+def test_both_sides_of_the_lines(rf, dev, seq, nq, nkv, causal):
+    q, k, v = inputs(seq, nq, nkv, seed=17)
+    scale = 1.0 / math.sqrt(D)
+    got = run(rf, q, k, v, causal, scale)
+    ref, mag = reference(q, k, v, causal, scale)
+    assert bool(((got - ref).abs() <= 1.25 * U16 * mag + 1e-5).all())      # as above
