@@ -2058,10 +2058,12 @@ void rf_attn_prefill_kernel(const _Float16* __restrict__ Q, const _Float16* __re
             const float alpha = __builtin_amdgcn_exp2f(m - m_new);
             m = m_new;
             l *= alpha;
+            if (it > 0) {                        // (O is zero before)
 #pragma unroll
-            for (int b = 0; b < 4; ++b)
+                for (int b = 0; b < 4; ++b)
 #pragma unroll
-                for (int e = 0; e < 16; ++e) o[b][e] *= alpha;
+                    for (int e = 0; e < 16; ++e) o[b][e] *= alpha;
+            }
             far = __builtin_amdgcn_ballot_w64(fabsf(m) >= kAttFar);
             if (far) {
 #pragma unroll
