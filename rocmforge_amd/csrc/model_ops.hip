@@ -1896,6 +1896,15 @@ constexpr uint32_t kAttRow = 2 * kAttD;          // bytes of a K / V row in LDS
 constexpr uint32_t kAttTile = 64 * kAttRow;      // one 64-key tile of K or of V
 constexpr float kAttFar = 128.0f;                // |m| from which scores are rounded before the exp
 
+// fmaxf of values that are no signalling NaNs, as one instruction: where the compiler
+// cannot know that, it quiets both operands first, a serial chain between the scores
+// and their exps (32 / 8 heads, 4096 positions 150.3 / 149.6 us, 8192 563 / 558).
+__device__ __forceinline__ float max_raw(float a, float b) {
+    float r;
+    asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+
 // NW waves as NW / KS units times KS key groups: group g takes the tiles
 // t % KS == g and the groups' partial (m, l, O) are merged through LDS (more
 // waves and a shorter walk per unit when the units are few).  VE: the V
@@ -2044,7 +2053,8 @@ void rf_attn_prefill_kernel(const _Float16* __restrict__ Q, const _Float16* __re
         for (int b = 0; b < 2; ++b)
 #pragma unroll
             for (int e = 0; e < 16; ++e) tmax = fmaxf(tmax, s[b][e]);
-        tmax = fmaxf(tmax, lane_xor<32>(tmax)) * scale2;
+        const auto halves = __builtin_amdgcn_permlane32_swap(__float_as_uint(tmax), __float_as_uint(tmax), false, false);
+        tmax = max_raw(__uint_as_float(halves[0]), __uint_as_float(halves[1])) * scale2;
         // O is rescaled only where some lane's maximum moved.  (A maximum left behind
         // by up to 2^8 saves 6 % of the time, but then a row's largest weight is no
         // longer exactly one and peaked rows lose half their precision.)
@@ -2054,7 +2064,7 @@ void rf_attn_prefill_kernel(const _Float16* __restrict__ Q, const _Float16* __re
         // zero the scores are rounded as m is (in this branch, taken on every tile then).
         float mul = scale2;
         if (__builtin_amdgcn_ballot_w64(tmax > m) | far) {
-            const float m_new = fmaxf(m, tmax);
+            const float m_new = max_raw(m, tmax);
             const float alpha = __builtin_amdgcn_exp2f(m - m_new);
             m = m_new;
             l *= alpha;
