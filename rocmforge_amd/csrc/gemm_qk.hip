@@ -12,18 +12,19 @@
 // own into library-owned device memory (the same values the reference's
 // __float2half gives) and run the fp16-activation tiles:
 //  * rf_gemm_q4k_f16a_kernel (Q4_K from 129 rows on where 256 x 128 tiles fill
-//    more than half of the CUs): 4 waves, each weight dequantised once per 256 rows of A,
-//    A and the weight ring by LDS DMA.
+//    more than half of the CUs): 4 waves, each weight dequantised once per 256
+//    rows of A, A and the weight ring by LDS DMA.
 //  * rf_gemm_q4k_f16s_kernel / rf_gemm_q4k_f16w_kernel (Q4_K otherwise) and
 //    rf_gemm_q6k_f16a_kernel (Q6_K from K = 768): 8 waves (mostly 16 on Q4_K's
-//    64-row tiles) over 64- to 256-row x 64-column tiles, K
-//    sliced over waves and added through LDS; when the tiles leave at least
-//    half the CUs idle, K is also split over workgroups whose partial tiles
+//    64-row tiles) over 64- to 256-row x 64-column tiles, K sliced over waves
+//    and added through LDS; when the tiles leave at least half the CUs idle, K
+//    is also split over workgroups whose partial tiles
 //    rf_gemm_split_reduce_kernel adds in split order.
 // Every output is one fixed-order sum: no float atomics, the same bits on
-// every run.  When no staging memory is free for the stream (or Q6_K weights
-// are not 16-byte aligned, or K is 256 or 512 with them) the fp32-activation
-// kernels run, one workgroup per tile:
+// every run.  When no staging memory is free for the stream, and for Q6_K
+// weights off a 16-byte address or with K = 256 or 512 (with K % 2048 != 0
+// also for an output off one), the fp32-activation kernels run, one workgroup
+// per tile:
 //  * rf_gemm_qk_sq_kernel (N % 256 == 0, K % 512 == 0, and 256 x 256 or
 //    128 x 128 tiles that come to about one workgroup per CU): 2 x 2 waves,
 //    each weight dequantised once per workgroup into an LDS B tile shared by
@@ -3621,7 +3622,7 @@ extern "C" hipError_t rf_gemm_q6_k_segments_launch(const float* input, const voi
 // launch (rf_gemm_f16_segs_kernel), each Q4_K (type 12) or Q6_K (type 14):
 // out_s[M x n_s] = fp16(A) * fp16(dequant W_s)^T, the products of
 // rf_gemm_q4_k_f16_launch / rf_gemm_q6_k_f16_launch on K-sliced 64-column
-// tiles of 128 or 256 rows.  The
+// tiles of 128 or 256 rows (their bits where they take such tiles unsplit).  The
 // prefill Q/K/V of a layer whatever its type mix.  M % 64, n_s % 64 (n1, n2
 // may be 0: fewer segments), K % 256 (K % 2048 with a Q6_K segment); input,
 // weights and outputs 16-byte aligned.

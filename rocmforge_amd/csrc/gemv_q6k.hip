@@ -196,7 +196,7 @@ __global__ __launch_bounds__(NW * 64) void rf_q6k_gemv_kernel(const uint8_t* __r
         y[row_begin + j] = out_lds[j] + (residual ? residual[row_begin + j] : 0.0f);
 }
 
-// ── K-split Q6_K GEMV with x held in registers (other K <= 16384) ───────────────
+// ── K-split Q6_K GEMV with x held in registers, direct loads (K <= 16384) ──────
 // A workgroup has one wave per 8-super-block slice of K (NWK = nsb/8
 // rounded up, at most 8 waves: K <= 16384).  The 8 lanes p = 0..7 of a
 // super-block sb = 8w + l/8 read its bytes with three 16-byte loads each,

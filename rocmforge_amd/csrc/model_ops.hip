@@ -593,9 +593,10 @@ __global__ __launch_bounds__(256) void rf_attn_decode_kernel(float* __restrict__
 // Split decode attention (the path used when the GQA group is at most 8
 // query heads).  Bound: up to a few thousand positions the two launches and
 // one trip to memory; beyond, the K / V stream and the VALU beside it (each
-// position and head takes 256 FMAs, on fp16 operands at half rate).  Grid = (kv head, split); a workgroup has one wave per
-// query head of the kv head's group, so the group's K/V rows are read once
-// per workgroup (the other waves hit L1).  Positions go out in chunks of
+// position and head takes 256 FMAs, on fp16 operands at half rate).  Grid =
+// (kv head, split); a workgroup has one wave per query head of the kv head's
+// group, so the group's K/V rows are read once per workgroup (the other waves
+// hit L1).  Positions go out in chunks of
 // kSplitChunk, chunk c to split c mod S, each wave keeping an online
 // (m, l, acc) over its chunks.  Within a chunk a wave issues all its K and
 // V loads (LPP lanes x 16 bytes per position, 64 / LPP positions per

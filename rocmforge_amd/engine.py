@@ -512,7 +512,7 @@ class Engine:
                         _chk(L.convert_f32_to_f16(_p(b[src]), _p(b[dst]), mp * c.kv_size, st), "to f16")
                     k16, v16 = b["k16"], b["v16"]
             # a Q4_K O projection reads the attention output as fp16 (the operand its
-            # fp32 launcher would round it to) through the K-sliced 128 x 64 tiles
+            # fp32 launcher would round it to)
             self._att16 = (self.fuse_gemm and self.ffn_f16 and m["attn_output"][1].wtype == GgmlType.Q4_K
                            and c.hidden % 64 == 0 and c.q_size % 256 == 0)
             if self._att16:
