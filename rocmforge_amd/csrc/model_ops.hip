@@ -609,11 +609,11 @@ constexpr int kSplitChunk = 32;
 // and, at D = 128 with two query heads or more to a KV head, the chunks come
 // through an LDS ring (use_long): the walk over a chunk at a time waited for
 // each chunk's loads, read every row once per head and spent a third of its
-// VALU on exps that 16 lanes computed alike.  32 / 8 heads, both launches, us
-// before / after (caches beyond the Infinity Cache): 16200 positions
-// 31.5 / 23.4, 8192 (40 heads) 30.1 / 27.6, 32000 (64 heads) 85.5 / 55.8; at
-// 4096, two rounds, 14.1 / 14.5; with one head to a KV head the direct walk is
-// as fast (4500 positions 14.0 against 17.6).
+// VALU on exps that 16 lanes computed alike.  32 / 8 heads, both launches from
+// a graph, us before / after (caches beyond the Infinity Cache): 6500 positions
+// 16.3 / 14.3, 16200 29.2 / 22.1, 8192 (40 heads) 19.7 / 17.2, 32000 (64 heads)
+// 71 / 44; at 4096, two rounds, the ring was no faster (14.1 / 14.5 in another
+// run), nor with one head to a KV head (4500 positions 14.0 / 17.6).
 constexpr int kLongRounds = 3;
 // Three stages are 48 KB, so three workgroups fit a CU beside the tables and a
 // grid of a few more than two a CU (S is rounded up: 520 at 10, 20 or 40 KV heads)
@@ -1880,9 +1880,9 @@ extern "C" hipError_t gpu_increment_decode_state_on_stream(int* d_state, hipStre
 // Bound: a 64-key tile is 32 MFMAs (1024 matrix cycles) against ~900 cycles
 // of softmax VALU per wave (32 v_exp_f32 at quarter rate, and an fma, an add
 // and half a max and a conversion per score), which overlap only across the
-// two waves of a SIMD.  32 / 8 heads, causal, fp16 output, graph replays, us
-// (TFLOP/s): 512 positions 17.2 -> 11.1, 1024 31.3 -> 23.2, 2048 110 -> 50
-// (686), 4096 420 -> 149 (920), 8192 1341 -> 552 (996).  Before: one wave
+// two waves of a SIMD.  32 / 8 heads, causal, fp16 output, graph replays on one
+// box, us (TFLOP/s): 512 positions 16.8 -> 10.3, 1024 30.9 -> 22.1, 2048 111 -> 50
+// (687), 4096 422 -> 157 (875), 8192 1356 -> 582 (945).  Before: one wave
 // per SIMD over 128 queries of one head, tiles through registers, V
 // transposed by 2-byte LDS stores.
 namespace rf {
