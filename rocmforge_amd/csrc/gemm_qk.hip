@@ -2542,7 +2542,7 @@ __device__ __forceinline__ void q4s_wg(const uint16_t* __restrict__ A, const uin
 // of an output are added through LDS in slice order, each output written
 // once.  A: the step's two 64-wide chunks (XOR-swizzled 128-byte rows), six
 // buffers; weights: three super-block stages, as there.
-// Measured (us, eight waves / sixteen, fp16 A, one box): 64 x 14336 x 4096
+// Measured (us, eight waves / sixteen, fp16 A, one run): 64 x 14336 x 4096
 // 23.6 / 21.3, 64 x 4096 x 12288 22.6 / 20.8, 64 x 8448 x 3072 accumulating
 // 18.4 / 15.7, 256 x 4096 x 11264 49.1 / 45.9.  Bound now: per super-block and
 // SIMD ~1300 cycles of VALU (65 instructions a wave, the 16 v_fma_mix at half

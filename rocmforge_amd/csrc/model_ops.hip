@@ -1880,8 +1880,8 @@ extern "C" hipError_t gpu_increment_decode_state_on_stream(int* d_state, hipStre
 // Bound: a 64-key tile is 32 MFMAs (1024 matrix cycles) against ~900 cycles
 // of softmax VALU per wave (32 v_exp_f32 at quarter rate, and an fma, an add
 // and half a max and a conversion per score), which overlap only across the
-// two waves of a SIMD.  32 / 8 heads, causal, fp16 output, graph replays on one
-// box, us (TFLOP/s): 512 positions 16.8 -> 10.3, 1024 30.9 -> 22.1, 2048 111 -> 50
+// two waves of a SIMD.  32 / 8 heads, causal, fp16 output, graph replays of
+// one run, us (TFLOP/s): 512 positions 16.8 -> 10.3, 1024 30.9 -> 22.1, 2048 111 -> 50
 // (687), 4096 422 -> 157 (875), 8192 1356 -> 582 (945).  Before: one wave
 // per SIMD over 128 queries of one head, tiles through registers, V
 // transposed by 2-byte LDS stores.
