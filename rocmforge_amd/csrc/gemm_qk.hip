@@ -2947,18 +2947,22 @@ static unsigned stream_grid(size_t n4) { return (unsigned)std::min<size_t>((n4 +
 constexpr int kGemmSlots = 4;
 constexpr size_t kSlotABytes = (size_t)32 << 20;
 constexpr size_t kSlotPartBytes = (size_t)24 << 20;
-constexpr size_t kSlotBytes = kSlotABytes + kSlotPartBytes;
-// The slots start at an odd multiple of 256 bytes (memory channels change every 256):
-// callers' matrices lie on multiples of 512, and with the staged A and the partials on
-// those too the Q6_K launches are 0.6-1.8 % slower (512 x 4096 x 14336 89.5 / 89.0 us,
-// 960 x 5120 x 13824 269.9 / 265.0; any odd multiple alike, Q4_K indifferent).  The
-// array's own place follows the code around it, hence the fixed offset in a page.
-constexpr size_t kSlotPage = 4096, kSlotPhase = 0x700;
-static __device__ __align__(256) uint8_t gemm_scratch[kGemmSlots * kSlotBytes + 2 * kSlotPage];
+// Memory channels change every 256 bytes and callers' matrices lie on multiples of
+// 512, so the staged A starts at an odd multiple of 256 and the partials at an even
+// one, whatever the array's address (it follows the code around it): fixed offsets in
+// a page.  us, weights from HBM, both even / both odd / this: Q6_K on fp32 A 512 x 4096 x
+// 14336 91.2 / 89.4 / 89.6, 960 x 5120 x 13824 271.5 / 265.4 / 265.4, 512 x 3584 x 18944
+// 111.5 / 108.4 / 108.1; Q4_K on fp16 A, split in eight, 64 x 2048 x 8192 14.29 / 14.60 /
+// 14.39, Q6_K adding 64 x 4096 x 14336 27.51 / 27.81 / 27.49; the rest alike.
+constexpr size_t kSlotPage = 4096, kSlotAPhase = 0x700;
+constexpr size_t kSlotBytes = kSlotABytes + kSlotPartBytes + kSlotPage;
+static_assert(kSlotBytes % kSlotPage == 0, "every slot starts a page");
+static __device__ __align__(256) uint8_t gemm_scratch[kGemmSlots * kSlotBytes + kSlotPage];
 constexpr int kGemmMaxDevices = 64;
 
 struct GemmSlot {
-    uint16_t* a;        // the slot's kSlotBytes
+    uint8_t* base;      // the slot's kSlotBytes
+    uint16_t* a() const { return reinterpret_cast<uint16_t*>(base + kSlotAPhase); }
 };
 
 // Room for K-split partials: the whole slot on the fp16-activation
@@ -2969,8 +2973,8 @@ struct PartBuf {
     size_t bytes;
 };
 static PartBuf slot_parts(const GemmSlot& slot, size_t a_bytes) {
-    const size_t off = (a_bytes + 255) & ~(size_t)255;
-    return PartBuf{reinterpret_cast<float*>(reinterpret_cast<uint8_t*>(slot.a) + off), kSlotBytes - off};
+    const size_t off = a_bytes == 0 ? 0 : (kSlotAPhase + a_bytes + 511) & ~(size_t)511;
+    return PartBuf{reinterpret_cast<float*>(slot.base + off), kSlotBytes - off};
 }
 
 struct SlotState {
@@ -2995,7 +2999,7 @@ static bool gemm_slot(hipStream_t st, GemmSlot* out) {
         void* p = nullptr;
         if (hipGetSymbolAddress(&p, HIP_SYMBOL(gemm_scratch)) != hipSuccess || p == nullptr) return false;
         const uintptr_t page = (reinterpret_cast<uintptr_t>(p) + kSlotPage - 1) / kSlotPage * kSlotPage;
-        g_slot_base[dev] = reinterpret_cast<uint8_t*>(page + kSlotPhase);
+        g_slot_base[dev] = reinterpret_cast<uint8_t*>(page);
     }
     SlotState* sl = g_slots[dev];
     int k = -1;
@@ -3009,8 +3013,7 @@ static bool gemm_slot(hipStream_t st, GemmSlot* out) {
     sl[k].taken = true;
     sl[k].owner = st;
     sl[k].captured = sl[k].captured || capturing;
-    uint8_t* b = g_slot_base[dev] + (size_t)k * kSlotBytes;
-    out->a = reinterpret_cast<uint16_t*>(b);
+    out->base = g_slot_base[dev] + (size_t)k * kSlotBytes;
     return true;
 }
 
@@ -3294,8 +3297,8 @@ static hipError_t staged_rows(const float* A, int M, int K, const GemmSlot& slot
         const int rows = std::min(run, M - m0);
         const size_t n4 = (size_t)rows * K / 4;
         hipLaunchKernelGGL(rf_f32_to_f16_kernel, dim3(stream_grid(n4)), dim3(256), 0, st,
-                           reinterpret_cast<const float4*>(A + (size_t)m0 * K), reinterpret_cast<uint2*>(slot.a), n4);
-        const hipError_t e = fn(slot.a, m0, rows, slot_parts(slot, (size_t)rows * K * 2));
+                           reinterpret_cast<const float4*>(A + (size_t)m0 * K), reinterpret_cast<uint2*>(slot.a()), n4);
+        const hipError_t e = fn(slot.a(), m0, rows, slot_parts(slot, (size_t)rows * K * 2));
         if (e != hipSuccess) return e;
     }
     return hipGetLastError();
