@@ -3147,16 +3147,24 @@ static void q4_f16_tiles(const uint16_t* A, const uint8_t* w, float* D, int M, i
                          const float* G, const PartBuf& part, const RowNorm* rn = nullptr) {
     const long tiles = (long)((M + 32 * FMR - 1) / (32 * FMR)) * (N / kQ4sBN);
     const int S = 2 * tiles <= (long)device_cu_count() ? ksplit_count(tiles, K / kQK, M, N, part) : 1;
-    // 64-row tiles split over K: sixteen waves where a workgroup's range is long enough
-    // to pay for filling their deeper pipeline and for adding eight partials in place
-    // of four (us, eight / sixteen waves, super-blocks a workgroup in brackets:
-    // 64 x 512 x 1024 [1] 9.1 / 9.5, 192 x 512 x 2560 [1] 11.2 / 12.0, 64 x 512 x 4096
-    // [2] 11.3 / 11.7, [3] 1-2 % slower, [4] alike, from [5] on 2-10 % faster; with more
-    // than 1024 rows A's traffic counts, 2048 x 256 x 2560 [5] 14.9 / 15.4, [8] alike).
-    // Unsplit always: storing they lose 1-3 % at one or two super-blocks and on
-    // 2048 x 512 up to K = 2560 (13.4 / 13.9 at 1536), accumulating, which takes the
-    // same tiles for the same bits, they gain 12-25 % there, and elsewhere both gain.
-    auto wide16 = [&](int S) { return FMR == 2 && (S == 1 || K / kQK / S >= (M > 1024 ? 8 : 5)); };
+    // 64-row tiles split over K: sixteen waves from four super-blocks a workgroup on, to
+    // pay for filling their deeper pipeline and for adding eight partials in place of
+    // four.  Eight-wave time over sixteen-wave time by super-blocks a workgroup, weights
+    // from HBM (in brackets from the Infinity Cache): [1] 0.97-1.02 (0.93-0.98), [2]
+    // 0.99-1.03 (0.95-0.99), [3] 0.98-1.03 (0.96-1.03), [4] 1.00-1.06 (0.98-1.04), [5] to
+    // [8] 1.00-1.06 (1.00-1.05).  With more than 1024 rows and (nearly) every CU taken A's
+    // traffic counts and five to seven are slower on sixteen: 2048 x 256 x 2560 15.5 / 14.9
+    // us, 4096 x 64 x 6144 16.2 / 15.6, 2048 x 128 x 6144 16.3 / 15.6; at [4] and [8] they
+    // are level or faster there too, and with CUs to spare at [5] as well (1088 x 256 x 4096,
+    // 204 workgroups, 13.3 / 14.0).  Unsplit always: storing they lose 1-3 % at one or two
+    // super-blocks and on 2048 x 512 up to K = 2560 (13.4 / 13.9 at 1536), accumulating,
+    // which takes the same tiles for the same bits, they gain 12-25 % there, and elsewhere
+    // both gain.
+    auto wide16 = [&](int S) {
+        const int per = K / kQK / S;
+        const bool crowded = M > 1024 && 16 * tiles * S >= 15L * device_cu_count();
+        return FMR == 2 && (S == 1 || per == 4 || per >= (crowded ? 8 : 4));
+    };
     auto go = [&](auto accc, float* d, const float* g, const KSplit& sp) {
         constexpr bool kAcc = decltype(accc)::value;
         const dim3 grid((unsigned)(tiles * sp.S));

@@ -51,9 +51,13 @@ def test_store_accumulate_and_swiglu(rf, dev, m, n, k):
 
 # Short ranges of a K split stay on eight waves with four K slices, as the segment
 # launcher's tiles take them: its products of the ranges, added in order, have the
-# same bits (these few tiles are split into single super-blocks, or pairs)
-@pytest.mark.parametrize("m,n,k,split", [(64, 64, 512, 2), (64, 192, 768, 3), (128, 64, 1024, 4), (64, 128, 4096, 8)])
+# same bits (these few tiles are split into one to three super-blocks; 128 tiles, with
+# 256 CUs, in two of five)
+@pytest.mark.parametrize("m,n,k,split", [(64, 64, 512, 2), (64, 192, 768, 3), (128, 64, 1024, 4), (64, 128, 4096, 8),
+                                         (64, 64, 6144, 8), (2048, 256, 2560, 2)])
 def test_short_k_ranges_on_eight_waves(rf, dev, m, n, k, split):
+    if m > 1024 and torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("split for 256 CUs")
     a = synth.activations(k, seed=m + n, m=m).astype(np.float16)
     w = synth.weights("q4_k", n, k, seed=k).reshape(n, k // 256, -1)
     z = None
@@ -70,3 +74,19 @@ def test_short_k_ranges_on_eight_waves(rf, dev, m, n, k, split):
     da, dw = G.to_dev(a.view(np.int16)), G.to_dev(w.reshape(-1))
     G.call(rf.rf_gemm_q4_k_f16_launch, G.ptr(da), G.ptr(dw), G.ptr(d), m, n, k)
     np.testing.assert_array_equal(G.host(d).reshape(m, n), want)
+
+
+# and from four super-blocks a workgroup on sixteen, with eight K slices: 64 rows of a
+# product have the bits of one too few tiles wide to be split otherwise
+@pytest.mark.parametrize("k", [8192, 8448])
+def test_longer_k_ranges_keep_their_bits(rf, dev, k):
+    a = synth.activations(k, seed=k, m=64).astype(np.float16)
+    w = synth.weights("q4_k", 128, k, seed=k + 1)
+    da, dw = G.to_dev(a.view(np.int16)), G.to_dev(w)
+    wide, narrow = G.empty(64 * 128, torch.float32), G.empty(64 * 64, torch.float32)
+    G.call(rf.rf_gemm_q4_k_f16_launch, G.ptr(da), G.ptr(dw), G.ptr(wide), 64, 128, k)
+    G.call(rf.rf_gemm_q4_k_f16_launch, G.ptr(da), G.ptr(dw), G.ptr(narrow), 64, 64, k)
+    got, ref = G.host(wide).reshape(64, 128), O.gemm("q4_k", a.astype(np.float32), w, 64, 128, k)
+    np.testing.assert_array_equal(got[:, :64], G.host(narrow).reshape(64, 64))
+    tol = 2e-3 * np.abs(ref) + 2e-5 * O.gemm_abs("q4_k", a.astype(np.float32), w, 64, 128, k)
+    assert (np.abs(got - ref) <= tol).all()
